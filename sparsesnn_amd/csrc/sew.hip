@@ -335,26 +335,42 @@ __global__ __launch_bounds__(kStemPix * 16 / CPT) void stem_conv_bn_lds_kernel(S
   }
 }
 
+// One neuron step of a hard-reset LIF / IF on charge h = fma(v, dec, x): the spike bit is shifted
+// into `word` from below (word = 2 word + spike) and v becomes vreset where it fired.
+__device__ __forceinline__ void stem_fire(float h, float vth, float vreset, float& v, uint32_t& word) {
+  asm("v_cmp_le_f32_e32 vcc, %[th], %[h]\n\t"
+      "v_cndmask_b32_e32 %[v], %[h], %[vr], vcc\n\t"
+      "v_addc_co_u32_e32 %[w], vcc, %[w], %[w], vcc"
+      : [v] "=&v"(v), [w] "+v"(word)
+      : [h] "v"(h), [th] "v"(vth), [vr] "v"(vreset)
+      : "vcc");
+}
+
 // Stem + neuron on the fp32 matrix cores (v_mfma_f32_16x16x4_f32, 4 taps per instruction):
-// the convolution as a GEMM of (output pixels) x (C_ * KH_ * KW_ taps, HWIO order: tap k =
-// (kh * KW + kw) * C + c, zero weights past the last tap) x (channels).  Workgroup = (image n,
-// 16 NB output pixels), NWV waves, wave w = channels 16w..16w+15 of all of them (NB 16-pixel
-// blocks, 4 NB accumulators per lane); the staged input rows are read by all waves.
-// Lane l supplies, per 4-tap step s, the input value of pixel l % 16 of each block at tap
-// 4s + l / 16 (the taps' staged-input offsets in an LDS table, its weights in registers) and
-// its weight for channel l % 16; it ends holding pixels 4 (l / 16) + r, r < 4, of each block for that channel.
-// Epilogue as in stem_conv_bn_lds_kernel<..., kStemSpikes, ...> (same BN, neuron arithmetic
-// and output layouts); a wave's 16-channel spike word of a pixel is the ballot of its spike
-// compare, picked out of the 64-lane mask by the lane that stores it.  The products are
-// summed in a different order than the FMA kernels', so outputs agree to fp32 rounding.
-// FASTN: hard-reset LIF with power-of-two 1/tau and 1 - 1/tau, or hard-reset IF, whose charge
-// is one fma (IF: v * 1 + x, the same single rounding as v + x); else the generic neuron.
-template <int C_, int KH_, int KW_, int NWV, bool FASTN, int NB>
-__global__ __launch_bounds__(64 * NWV) void stem_mfma_kernel(StemParams p) {
-  constexpr int NT = 64 * NWV;
+// the convolution as a GEMM of channels x (C_ * KH_ * KW_ taps, HWIO order: tap k =
+// (kh * KW + kw) * C + c, zero weights past the last tap) x (output pixels).  Workgroup = (image
+// n, PIX = 16 NB * 4 / NCG output pixels), four waves: wave w holds CT 16-channel tiles of the
+// w % NCG-th channel group for the 16 NB pixels of set w / NCG, so an input value read from LDS
+// feeds CT matrix instructions (one per wave before: the LDS reads and their address adds, and the
+// epilogue below, took as long as the products).  Lane l supplies, per 4-tap step s, the input
+// value of pixel l % 16 of each block at tap 4s + l / 16 (the taps' staged-input offsets in an LDS
+// table) and its weight for channel l % 16 (registers); it ends holding channels 4 (l / 16) + r,
+// r < 4, of each tile for pixel l % 16.
+// Epilogue: BN, one 16-byte store per tile where the fp32 output is kept, and the neuron over four
+// timesteps at a time: a lane's 4 channels x 4 steps are a 16-bit word of nibbles, two tiles share a
+// register, and a 4 x 4 nibble transpose among the lanes of a pixel (two butterfly steps) leaves
+// lane l with the whole channel words of one timestep: one store per tile pair for four steps.
+// The products are summed in a different order than the FMA kernels', so outputs agree to fp32
+// rounding.  FASTN: hard-reset LIF with power-of-two 1/tau and 1 - 1/tau, or hard-reset IF, whose
+// charge is one fma (IF: v * 1 + x, the same single rounding as v + x); else the generic neuron.
+// 7x7/2 224x224, 64 channels, T = 4, fp32 output kept: 8 images 44.0 -> 34.6 us, 32 images
+// 114.9 -> 110.1; 3x3 224x224, spikes only, 32 images: 171.9 -> 124.4.
+template <int C_, int KH_, int KW_, int CT, int NCG, bool FASTN, int NB>
+__global__ __launch_bounds__(256) void stem_mfma_kernel(StemParams p) {
+  constexpr int NT = 256;
   constexpr int K = C_ * KH_ * KW_;
   constexpr int KS = (K + 3) / 4;
-  constexpr int PIX = 16 * NB;  // output pixels per workgroup
+  constexpr int PIX = 16 * NB * (4 / NCG);  // output pixels per workgroup
   // LDS: the staged-input offsets of the 4 KS taps (int), then the staged input rows
   extern __shared__ float lds_stem[];
   int* const sk = reinterpret_cast<int*>(lds_stem);
@@ -372,12 +388,14 @@ __global__ __launch_bounds__(64 * NWV) void stem_mfma_kernel(StemParams p) {
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int q = lane >> 4, j = lane & 15;
-  const int ch = wv * 16 + j;
-  float wb[KS];
+  const int ch0 = (wv % NCG) * 16 * CT;  // the wave's first channel
+  const int wpix0 = pix0 + (wv / NCG) * 16 * NB;
+  float wb[CT][KS];
 #pragma unroll
   for (int s = 0; s < KS; ++s) {
     const int k = 4 * s + q;
-    wb[s] = k < K ? p.w[(int64_t)k * p.F + ch] : 0.f;
+#pragma unroll
+    for (int c = 0; c < CT; ++c) wb[c][s] = k < K ? p.w[(int64_t)k * p.F + ch0 + 16 * c + j] : 0.f;
   }
   for (int k = threadIdx.x; k < 4 * KS; k += NT) {
     const int kk = k < K ? k : K - 1;  // a real tap of the same pixel; its weight is zero
@@ -386,18 +404,20 @@ __global__ __launch_bounds__(64 * NWV) void stem_mfma_kernel(StemParams p) {
   }
   stem_stage_rows<NT>(p, sx, p.x + (int64_t)n * C_ * p.H * p.W, ih0, nrows, WP);
   __syncthreads();
-  // Pixel pix0 + 16 b + j of block b (past the image: pixel pix0, computed but not stored).
+  // Pixel wpix0 + 16 b + j of block b (past the image: its last pixel, computed but not stored).
   // Every staged offset read is below C * nrows * WP: (OW - 1) * SW + KW - 1 < W + 2 * PW.
   int base[NB];
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
-    const int pix = min(pix0 + 16 * b + j, npix - 1);
+    const int pix = min(min(wpix0 + 16 * b + j, npix - 1), pix0 + PIX - 1);
     const int oh = pix / p.OW;
     base[b] = (oh - oh_first) * p.SH * WP + (pix - oh * p.OW) * p.SW;
   }
-  float4_t acc[NB];
+  float4_t acc[NB][CT];
 #pragma unroll
-  for (int b = 0; b < NB; ++b) acc[b] = float4_t{0.f, 0.f, 0.f, 0.f};
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int c = 0; c < CT; ++c) acc[b][c] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < KS; ++s) {
     const int koff = sk[4 * s + q];
@@ -405,40 +425,87 @@ __global__ __launch_bounds__(64 * NWV) void stem_mfma_kernel(StemParams p) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) a[b] = sx[base[b] + koff];
 #pragma unroll
-    for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[b], wb[s], acc[b], 0, 0, 0);
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+        acc[b][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(wb[c][s], a[b], acc[b][c], 0, 0, 0);
   }
-  const float sc = p.scale[ch], bi = p.bias[ch];
   const bool fold = p.np.neuron == SENGINE_NEURON_LIF && p.np.pow2;
   const float dec = p.np.neuron == SENGINE_NEURON_IF ? 1.f : p.np.decay;
   const int fw = p.F / 16;
   const int64_t tstride = (int64_t)p.N * npix * fw;
-  // the word this lane stores (lanes 0-15): pixel 4 g + r of a block, g = j / 4, r = j % 4
-  const int rsel = j & 3, gsh = 16 * (j >> 2);
+  typedef float out4_t __attribute__((ext_vector_type(4), aligned(4)));
+  float sc[CT][4], bi[CT][4];
 #pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    float xo[4], v[4];
+  for (int c = 0; c < CT; ++c)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      xo[r] = __builtin_fmaf(acc[b][r], sc, bi);
-      const int pix = pix0 + 16 * b + 4 * q + r;
-      if (p.out && pix < npix) p.out[((int64_t)n * npix + pix) * p.F + ch] = xo[r];
-      if (fold) xo[r] *= p.np.rtau;  // exact
-      v[r] = 0.f;
+      sc[c][r] = p.scale[ch0 + 16 * c + 4 * q + r];
+      bi[c][r] = p.bias[ch0 + 16 * c + 4 * q + r];
     }
-    const int spix = pix0 + 16 * b + j;
-    uint16_t* so = p.spikes + ((int64_t)n * npix + spix) * fw + wv;
-    const bool st = q == 0 && spix < npix;
-    for (int t = 0; t < p.T; ++t) {
-      uint64_t mk[4];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const int pix = wpix0 + 16 * b + j;
+    const bool st = pix < npix;
+    const int64_t opix = (int64_t)n * npix + pix;
+    float xo[CT][4], v[CT][4];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float h = FASTN ? __builtin_fmaf(v[r], dec, xo[r]) : neuron_charge(p.np, v[r], xo[r]);
-        const bool spike = h >= p.np.vth;
-        v[r] = FASTN ? (spike ? p.np.vreset : h) : neuron_reset(p.np, h, spike);
-        mk[r] = __builtin_amdgcn_ballot_w64(spike);
+        xo[c][r] = __builtin_fmaf(acc[b][c][r], sc[c][r], bi[c][r]);
+        v[c][r] = 0.f;
       }
-      const uint64_t m = rsel == 0 ? mk[0] : rsel == 1 ? mk[1] : rsel == 2 ? mk[2] : mk[3];
-      if (st) so[t * tstride] = (uint16_t)(m >> gsh);
+      if (p.out && st)
+        *reinterpret_cast<out4_t*>(p.out + opix * p.F + ch0 + 16 * c + 4 * q) =
+            out4_t{xo[c][0], xo[c][1], xo[c][2], xo[c][3]};
+      if (fold) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) xo[c][r] *= p.np.rtau;  // exact
+      }
+    }
+    for (int t0 = 0; t0 < p.T; t0 += 4) {
+      uint32_t nib[CT];
+#pragma unroll
+      for (int c = 0; c < CT; ++c) nib[c] = 0u;
+#pragma unroll
+      for (int k = 0; k < 4; ++k)  // steps past T run and are not stored
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+          for (int r = 3; r >= 0; --r) {
+            if (FASTN) {
+              stem_fire(__builtin_fmaf(v[c][r], dec, xo[c][r]), p.np.vth, p.np.vreset, v[c][r], nib[c]);
+            } else {
+              const float h = neuron_charge(p.np, v[c][r], xo[c][r]);
+              const bool spike = h >= p.np.vth;
+              v[c][r] = neuron_reset(p.np, h, spike);
+              nib[c] = 2 * nib[c] + (uint32_t)spike;
+            }
+          }
+      // nib: step t0 + k in nibble 3 - k.  Lane group q ends with step t0 + 3 - q, the nibble of
+      // source group g at bits 4g of the tile's 16.
+      const int t = t0 + 3 - q;
+      uint32_t wd[CT / 2];
+#pragma unroll
+      for (int c = 0; c < CT / 2; ++c) {
+        const uint32_t x = nib[2 * c] | (nib[2 * c + 1] << 16);
+        const uint32_t px = (uint32_t)__shfl_xor((int)x, 32, 64);
+        const uint32_t y = q < 2 ? (x & 0x00ff00ffu) | ((px & 0x00ff00ffu) << 8)
+                                 : (x & 0xff00ff00u) | ((px & 0xff00ff00u) >> 8);
+        const uint32_t py = (uint32_t)__shfl_xor((int)y, 16, 64);
+        wd[c] = (q & 1) == 0 ? (y & 0x0f0f0f0fu) | ((py & 0x0f0f0f0fu) << 4)
+                             : (y & 0xf0f0f0f0u) | ((py & 0xf0f0f0f0u) >> 4);
+      }
+      if (st && t < p.T) {
+        uint16_t* so = p.spikes + t * tstride + opix * fw + ch0 / 16;
+        if constexpr (CT == 4) {
+          typedef uint32_t w2_t __attribute__((ext_vector_type(2), aligned(4)));
+          *reinterpret_cast<w2_t*>(so) = w2_t{wd[0], wd[1]};
+        } else {
+          *reinterpret_cast<uint32_t*>(so) = wd[0];
+        }
+      }
     }
   }
 }
@@ -809,48 +876,52 @@ static int64_t stem_staged(const StemParams& p, int pix) {
 
 // Launch geometry of stem_mfma_kernel<..., NB>: workgroups, the rounds the chip needs for
 // them at the occupancy the kernel reaches (resident workgroups per CU x CUs), and its LDS.
-template <int K_, int NWV, bool FASTN, int NB>
+template <int K_, int CT, int NCG, bool FASTN, int NB>
 static void stem_mfma_shape(const StemParams& p, int cus, int64_t& wgs, int64_t& rounds, size_t& lds) {
-  lds = (size_t)(stem_staged(p, 16 * NB) + 4 * ((3 * K_ * K_ + 3) / 4)) * sizeof(float);  // + tap offsets
-  wgs = (int64_t)p.N * ((p.OH * p.OW + 16 * NB - 1) / (16 * NB));
+  constexpr int PIX = 16 * NB * (4 / NCG);
+  lds = (size_t)(stem_staged(p, PIX) + 4 * ((3 * K_ * K_ + 3) / 4)) * sizeof(float);  // + tap offsets
+  wgs = (int64_t)p.N * ((p.OH * p.OW + PIX - 1) / PIX);
   int per_cu = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(
-                                                       &stem_mfma_kernel<3, K_, K_, NWV, FASTN, NB>),
-                                                   64 * NWV, lds) != hipSuccess ||
+                                                       &stem_mfma_kernel<3, K_, K_, CT, NCG, FASTN, NB>),
+                                                   256, lds) != hipSuccess ||
       per_cu < 1)
     per_cu = 1;
   const int64_t slots = (int64_t)per_cu * cus;
   rounds = (wgs + slots - 1) / slots;
 }
 
-// Pixels per workgroup (16 NB): the fewest pixel-block rounds over the chip, weighing a round
-// by its workgroup's pixels; at equal cost the larger block (less halo staging).
-template <int K_, int NWV, bool FASTN>
+// Pixels per workgroup (16 NB * 4 / NCG): the fewest pixel-block rounds over the chip, weighing a
+// round by its workgroup's pixels plus 64 for what every workgroup pays (staging, weights): without
+// that term the 32-image 7x7 stem took seven rounds of 128 pixels (117.8 us) over four of 256 (110.1).
+template <int K_, int CT, int NCG, bool FASTN>
 static int launch_stem_mfma(const StemParams& p, hipStream_t stream) {
+  constexpr int S = 4 / NCG;  // pixel sets per workgroup
+  constexpr int NL = 16 / S, NM = 12 / S, NS = 8 / S;  // 256, 192 or 128 pixels
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
                                                hipSuccess)
     cus = 256;
-  int64_t w16, r16, w11, r11, w8, r8;
-  size_t l16, l11, l8;
-  stem_mfma_shape<K_, NWV, FASTN, 16>(p, cus, w16, r16, l16);
-  stem_mfma_shape<K_, NWV, FASTN, 11>(p, cus, w11, r11, l11);
-  stem_mfma_shape<K_, NWV, FASTN, 8>(p, cus, w8, r8, l8);
+  int64_t wl, rl, wm, rm, ws, rs;
+  size_t ll, lm, ls;
+  stem_mfma_shape<K_, CT, NCG, FASTN, NL>(p, cus, wl, rl, ll);
+  stem_mfma_shape<K_, CT, NCG, FASTN, NM>(p, cus, wm, rm, lm);
+  stem_mfma_shape<K_, CT, NCG, FASTN, NS>(p, cus, ws, rs, ls);
   int nb = 16;
-  int64_t best = r16 * 16;
-  if (r11 * 11 < best) { nb = 11; best = r11 * 11; }
-  if (r8 * 8 < best) nb = 8;
+  int64_t best = rl * (16 + 4);
+  if (rm * (12 + 4) < best) { nb = 12; best = rm * (12 + 4); }
+  if (rs * (8 + 4) < best) nb = 8;
   if (const char* e = getenv("SENGINE_AMD_STEM_NB")) {
     const int f = atoi(e);
-    if (f == 16 || f == 11 || f == 8) nb = f;
+    if (f == 16 || f == 12 || f == 8) nb = f;
   }
-  const dim3 block(64 * NWV);
+  const dim3 block(256);
   if (nb == 16)
-    hipLaunchKernelGGL((stem_mfma_kernel<3, K_, K_, NWV, FASTN, 16>), dim3((unsigned)w16), block, l16, stream, p);
-  else if (nb == 11)
-    hipLaunchKernelGGL((stem_mfma_kernel<3, K_, K_, NWV, FASTN, 11>), dim3((unsigned)w11), block, l11, stream, p);
+    hipLaunchKernelGGL((stem_mfma_kernel<3, K_, K_, CT, NCG, FASTN, NL>), dim3((unsigned)wl), block, ll, stream, p);
+  else if (nb == 12)
+    hipLaunchKernelGGL((stem_mfma_kernel<3, K_, K_, CT, NCG, FASTN, NM>), dim3((unsigned)wm), block, lm, stream, p);
   else
-    hipLaunchKernelGGL((stem_mfma_kernel<3, K_, K_, NWV, FASTN, 8>), dim3((unsigned)w8), block, l8, stream, p);
+    hipLaunchKernelGGL((stem_mfma_kernel<3, K_, K_, CT, NCG, FASTN, NS>), dim3((unsigned)ws), block, ls, stream, p);
   return (int)hipGetLastError();
 }
 
@@ -930,11 +1001,16 @@ extern "C" int sengine_amd_stem_conv_bn_neuron(const sengine_conv_lif_desc* d, c
   if (p.C == 3 && p.KH == p.KW && (p.KW == 7 || p.KW == 3) && (p.F == 32 || p.F == 64) && env_stem_mfma()) {
     const bool fast = p.np.hard_reset && (p.np.neuron == SENGINE_NEURON_IF ||
                                           (p.np.neuron == SENGINE_NEURON_LIF && p.np.pow2));
-    if (p.KW == 7)
-      return p.F == 64 ? (fast ? launch_stem_mfma<7, 4, true>(p, stream) : launch_stem_mfma<7, 4, false>(p, stream))
-                       : (fast ? launch_stem_mfma<7, 2, true>(p, stream) : launch_stem_mfma<7, 2, false>(p, stream));
-    return p.F == 64 ? (fast ? launch_stem_mfma<3, 4, true>(p, stream) : launch_stem_mfma<3, 4, false>(p, stream))
-                     : (fast ? launch_stem_mfma<3, 2, true>(p, stream) : launch_stem_mfma<3, 2, false>(p, stream));
+#define SENGINE_STEM_CASE(K, FF, CT, NCG) \
+  if (p.KW == K && p.F == FF)             \
+    return fast ? launch_stem_mfma<K, CT, NCG, true>(p, stream) : launch_stem_mfma<K, CT, NCG, false>(p, stream);
+    // channel tiles per wave: all of them where a tile's weights take few registers (3x3: 7),
+    // two for the 7x7 stem's 37
+    SENGINE_STEM_CASE(7, 64, 2, 2)
+    SENGINE_STEM_CASE(7, 32, 2, 1)
+    SENGINE_STEM_CASE(3, 64, 4, 1)
+    SENGINE_STEM_CASE(3, 32, 2, 1)
+#undef SENGINE_STEM_CASE
   }
   const int64_t blocks = pblocks * (p.F / 16);
   if (p.KW == 7)
