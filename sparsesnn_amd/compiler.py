@@ -15,7 +15,6 @@ runtime's (KH, KW, C_in, C_out) layout (cuda_graph_runtime.py:233-235) or torch'
 """
 from __future__ import annotations
 
-import dataclasses
 
 import numpy as np
 import torch
@@ -103,7 +102,7 @@ class FusedSparseConvBNLIFKernel:
         self.OH, self.OW, self.M, self.K_red = ops.geometry(spec)
 
     def spec_for(self, in_enc: int, out_enc: int) -> ConvSpec:
-        return dataclasses.replace(self.spec, in_enc=in_enc, out_enc=out_enc)
+        return self.spec.with_enc(in_enc, out_enc)
 
     def prepare_weight(self, w, device=None) -> SparseWeight:
         if self.in_planes > 1 and not isinstance(w, SparseWeight):
@@ -232,7 +231,7 @@ class DenseConvBNKernel:
         in_enc = ENC_BITS if data.dtype == torch.int32 else ENC_F16 if data.dtype == torch.float16 else None
         if in_enc is None:
             raise SEngineError("data must be fp16 NHWC or int32 spike bits")
-        spec = dataclasses.replace(self.spec, in_enc=in_enc)
+        spec = self.spec.with_enc(in_enc, self.spec.out_enc)
         if isinstance(weight, torch.Tensor) and weight.dtype == torch.int16:
             blob = weight
         else:

@@ -10,7 +10,7 @@ from __future__ import annotations
 import ctypes
 import math
 import os
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 from typing import Optional
 
 import torch
@@ -31,11 +31,22 @@ __all__ = [
 
 
 def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # absent in CPU-only builds
 
 
 def _stream(device: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """The device's current stream as an integer handle (no torch Stream object is made)."""
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
+
+
+def _fits(t, dtype: torch.dtype, numel: int) -> bool:
+    """Whether _require_cuda and _require_numel both accept t."""
+    return isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is dtype and t.numel() == numel and t.is_contiguous()
 
 
 def _require_cuda(t: torch.Tensor, name: str):
@@ -81,6 +92,119 @@ class ConvSpec:
 
     def desc(self) -> ConvLifDesc:
         return make_desc(self)
+
+    def __getstate__(self):
+        """The fields alone: what is derived from them (ctypes objects) is rebuilt where it is needed."""
+        return {k: v for k, v in self.__dict__.items() if not k.startswith("_")}
+
+    def with_enc(self, in_enc: int, out_enc: int) -> "ConvSpec":
+        """This spec with other encodings; made once per pair and kept, with its own plan."""
+        made = self.__dict__.get("_variants")
+        if made is None:
+            made = {}
+            object.__setattr__(self, "_variants", made)
+        v = made.get((in_enc, out_enc))
+        if v is None:
+            v = made[(in_enc, out_enc)] = replace(self, in_enc=in_enc, out_enc=out_enc)
+        return v
+
+
+def _ref(s: ConvSpec):
+    """The spec's C descriptor by reference (which keeps it alive), made once per spec."""
+    r = s.__dict__.get("_desc_ref")
+    if r is None:
+        r = ctypes.byref(make_desc(s))
+        object.__setattr__(s, "_desc_ref", r)
+    return r
+
+
+class _Plan:
+    """What every call derives from a ConvSpec alone: its C descriptor, geometry, blob sizes and
+    activation layouts.  A spec is immutable, so they are worked out once and kept on it (a call
+    spent more host time on them than on its launch)."""
+
+    __slots__ = ("ref", "OH", "OW", "M", "_blob", "_dense", "_in", "_out")
+
+    def __init__(self, s: "ConvSpec"):
+        lib = _lib.load()
+        self.ref = _ref(s)
+        oh, ow = ctypes.c_int32(), ctypes.c_int32()
+        m, k = ctypes.c_int64(), ctypes.c_int64()
+        check(lib.sengine_amd_conv_geometry(self.ref, ctypes.byref(oh), ctypes.byref(ow), ctypes.byref(m),
+                                            ctypes.byref(k)), "conv_geometry")
+        self.OH, self.OW, self.M = oh.value, ow.value, m.value
+        self._blob = self._dense = self._in = self._out = None
+
+    def blob(self):
+        """(value bytes, metadata bytes) of the sparse weight blob."""
+        if self._blob is None:
+            vb, mb = ctypes.c_size_t(), ctypes.c_size_t()
+            check(_lib.load().sengine_amd_sparse_blob_bytes(self.ref, ctypes.byref(vb), ctypes.byref(mb)),
+                  "sparse_blob_bytes")
+            self._blob = (vb.value, mb.value)
+        return self._blob
+
+    def dense_blob(self) -> int:
+        if self._dense is None:
+            vb = ctypes.c_size_t()
+            check(_lib.load().sengine_amd_dense_blob_bytes(self.ref, ctypes.byref(vb)), "dense_blob_bytes")
+            self._dense = vb.value
+        return self._dense
+
+    def data(self, s: "ConvSpec"):
+        """(dtype, numel) of the input."""
+        if self._in is None:
+            self._in = _enc_numel(s.in_enc, s.T * s.B * s.H * s.W * s.C_in)
+        return self._in
+
+    def spikes(self, s: "ConvSpec"):
+        """(dtype, numel, shape) of the output spikes."""
+        if self._out is None:
+            dt, n = _enc_numel(s.out_enc, s.T * self.M * s.C_out)
+            last = s.C_out // 32 if s.out_enc == ENC_BITS else s.C_out
+            self._out = (dt, n, (s.T * s.B, self.OH, self.OW, last))
+        return self._out
+
+
+def _plan(s: ConvSpec) -> _Plan:
+    p = s.__dict__.get("_plan")
+    if p is None:
+        p = _Plan(s)
+        object.__setattr__(s, "_plan", p)
+    return p
+
+
+def _check_fused(who: str, s: ConvSpec, p: _Plan, data, values, meta, bn_scale, bn_bias, extra=()):
+    """The checks shared by the fused calls: the input and the weight blob against the descriptor,
+    the BN vectors, and `extra` tensors that only have to be contiguous on the device."""
+    vb, mb = p.blob()
+    dt, n_in = p.data(s) if isinstance(data, torch.Tensor) and data.is_cuda else (None, 0)
+    if _fits(data, dt, n_in) and _fits(bn_scale, torch.float32, s.C_out) and _fits(bn_bias, torch.float32, s.C_out) \
+            and isinstance(values, torch.Tensor) and values.is_cuda and values.is_contiguous() and values.nbytes == vb \
+            and isinstance(meta, torch.Tensor) and meta.is_cuda and meta.is_contiguous() and meta.nbytes == mb \
+            and all(isinstance(t, torch.Tensor) and t.is_cuda and t.is_contiguous() for t, _ in extra):
+        return
+    for t, n in ((data, "data"), (values, "values"), (meta, "meta"), (bn_scale, "bn_scale"), (bn_bias, "bn_bias"),
+                 *extra):
+        _require_cuda(t, n)
+    dt, n_in = p.data(s)
+    _require_numel(data, n_in, dt, "data")
+    if values.numel() * values.element_size() != vb or meta.numel() * meta.element_size() != mb:
+        raise SEngineError(f"{who}: weight blob does not match the descriptor")
+    _require_numel(bn_scale, s.C_out, torch.float32, "bn_scale")
+    _require_numel(bn_bias, s.C_out, torch.float32, "bn_bias")
+
+
+def _check_req(t, numel: int, dtype: torch.dtype, name: str):
+    if not _fits(t, dtype, numel):
+        _require_cuda(t, name)
+        _require_numel(t, numel, dtype, name)
+
+
+def _check_opt(t, numel: int, dtype: torch.dtype, name: str):
+    """An optional buffer of a call (None passes)."""
+    if t is not None:
+        _check_req(t, numel, dtype, name)
 
 
 _NEURON_CODES = {"lif": NEURON_LIF, "if": NEURON_IF, "ms": NEURON_MS}
@@ -264,37 +388,20 @@ def fused_sparse_conv_bn_lif(s: ConvSpec, data: torch.Tensor, values: torch.Tens
     """Fused 2:4 Conv + BN + multi-step neuron (one launch).  Returns the spike tensor:
     bits int32 (T*B, OH, OW, C_out/32) or fp16 (T*B, OH, OW, C_out) per s.out_enc."""
     lib = _lib.load()
-    OH, OW, M, _ = geometry(s)
-    d = make_desc(s)
-    vb, mb = ctypes.c_size_t(), ctypes.c_size_t()
-    check(lib.sengine_amd_sparse_blob_bytes(ctypes.byref(d), ctypes.byref(vb), ctypes.byref(mb)), "sparse_blob_bytes")
-    for t, n in ((data, "data"), (values, "values"), (meta, "meta"), (bn_scale, "bn_scale"), (bn_bias, "bn_bias")):
-        _require_cuda(t, n)
+    p = _plan(s)
+    _check_fused("fused_sparse_conv_bn_lif", s, p, data, values, meta, bn_scale, bn_bias)
     dev = data.device
-    dt, n_in = _enc_numel(s.in_enc, s.T * s.B * s.H * s.W * s.C_in)
-    _require_numel(data, n_in, dt, "data")
-    if values.numel() * values.element_size() != vb.value or meta.numel() * meta.element_size() != mb.value:
-        raise SEngineError("fused_sparse_conv_bn_lif: weight blob does not match the descriptor")
-    _require_numel(bn_scale, s.C_out, torch.float32, "bn_scale")
-    _require_numel(bn_bias, s.C_out, torch.float32, "bn_bias")
-    if state is not None:
-        _require_cuda(state, "state")
-        _require_numel(state, M * s.C_out, torch.float32, "state")
-    for tr, n in ((h_trace, "h_trace"), (x_trace, "x_trace")):
-        if tr is not None:
-            _require_cuda(tr, n)
-            _require_numel(tr, s.T * M * s.C_out, torch.float32, n)
-    odt, n_out = _enc_numel(s.out_enc, s.T * M * s.C_out)
+    _check_opt(state, p.M * s.C_out, torch.float32, "state")
+    _check_opt(h_trace, s.T * p.M * s.C_out, torch.float32, "h_trace")
+    _check_opt(x_trace, s.T * p.M * s.C_out, torch.float32, "x_trace")
+    odt, n_out, shape = p.spikes(s)
     if out is None:
-        last = s.C_out // 32 if s.out_enc == ENC_BITS else s.C_out
-        out = torch.empty(s.T * s.B, OH, OW, last, dtype=odt, device=dev)
+        out = torch.empty(shape, dtype=odt, device=dev)
     else:
-        _require_cuda(out, "out")
-        _require_numel(out, n_out, odt, "out")
-    rc = lib.sengine_amd_fused_sparse_conv_bn_lif(
-        ctypes.byref(d), _ptr(data), _ptr(values), _ptr(meta), _ptr(state), _ptr(bn_scale), _ptr(bn_bias),
-        _ptr(out), _ptr(h_trace), _ptr(x_trace), _stream(dev))
-    check(rc, "fused_sparse_conv_bn_lif")
+        _check_opt(out, n_out, odt, "out")
+    check(lib.sengine_amd_fused_sparse_conv_bn_lif(
+        p.ref, data.data_ptr(), values.data_ptr(), meta.data_ptr(), _ptr(state), bn_scale.data_ptr(),
+        bn_bias.data_ptr(), out.data_ptr(), _ptr(h_trace), _ptr(x_trace), _stream(dev)), "fused_sparse_conv_bn_lif")
     return out
 
 
@@ -353,26 +460,15 @@ def fused_sparse_conv_bn_lif_split(s: ConvSpec, data: torch.Tensor, values: torc
     lib = _lib.load()
     if s.out_enc != ENC_BITS:
         raise SEngineError("fused_sparse_conv_bn_lif_split: spike-bit output only")
-    OH, OW, M, _ = geometry(s)
-    d = make_desc(s)
-    vb, mb = ctypes.c_size_t(), ctypes.c_size_t()
-    check(lib.sengine_amd_sparse_blob_bytes(ctypes.byref(d), ctypes.byref(vb), ctypes.byref(mb)), "sparse_blob_bytes")
-    for t, n in ((data, "data"), (values, "values"), (meta, "meta"), (bn_scale, "bn_scale"), (bn_bias, "bn_bias")):
-        _require_cuda(t, n)
-    dt, n_in = _enc_numel(s.in_enc, s.T * s.B * s.H * s.W * s.C_in)
-    _require_numel(data, n_in, dt, "data")
-    if values.numel() * values.element_size() != vb.value or meta.numel() * meta.element_size() != mb.value:
-        raise SEngineError("fused_sparse_conv_bn_lif_split: weight blob does not match the descriptor")
-    _require_numel(bn_scale, s.C_out, torch.float32, "bn_scale")
-    _require_numel(bn_bias, s.C_out, torch.float32, "bn_bias")
+    p = _plan(s)
+    _check_fused("fused_sparse_conv_bn_lif_split", s, p, data, values, meta, bn_scale, bn_bias)
     nplanes = -(-s.C_out // split)
     if out is None:
-        out = torch.empty(nplanes, s.T * s.B, OH, OW, split // 32, dtype=torch.int32, device=data.device)
+        out = torch.empty(nplanes, s.T * s.B, p.OH, p.OW, split // 32, dtype=torch.int32, device=data.device)
     else:
-        _require_cuda(out, "out")
-        _require_numel(out, nplanes * s.T * M * split // 32, torch.int32, "out")
+        _check_opt(out, nplanes * s.T * p.M * split // 32, torch.int32, "out")
     check(lib.sengine_amd_fused_sparse_conv_bn_lif_split(
-        ctypes.byref(d), _ptr(data), _ptr(values), _ptr(meta), None, _ptr(bn_scale), _ptr(bn_bias), _ptr(out), split,
+        p.ref, _ptr(data), _ptr(values), _ptr(meta), None, _ptr(bn_scale), _ptr(bn_bias), _ptr(out), split,
         _stream(data.device)), "fused_sparse_conv_bn_lif_split")
     return out
 
@@ -435,41 +531,26 @@ def fused_sparse_conv_bn_lif_add(s: ConvSpec, data: torch.Tensor, values: torch.
     f16 = s.out_enc == ENC_F16
     if s.out_enc != ENC_BITS and not f16:
         raise SEngineError("fused_sparse_conv_bn_lif_add: out_enc must be ENC_BITS or ENC_F16")
-    OH, OW, M, _ = geometry(s)
-    d = make_desc(s)
-    vb, mb = ctypes.c_size_t(), ctypes.c_size_t()
-    check(lib.sengine_amd_sparse_blob_bytes(ctypes.byref(d), ctypes.byref(vb), ctypes.byref(mb)), "sparse_blob_bytes")
-    for t, n in ((data, "data"), (values, "values"), (meta, "meta"), (bn_scale, "bn_scale"), (bn_bias, "bn_bias"),
-                 (residual, "residual")):
-        _require_cuda(t, n)
-    dev = data.device
-    dt, n_in = _enc_numel(s.in_enc, s.T * s.B * s.H * s.W * s.C_in)
-    _require_numel(data, n_in, dt, "data")
-    if values.numel() * values.element_size() != vb.value or meta.numel() * meta.element_size() != mb.value:
-        raise SEngineError("fused_sparse_conv_bn_lif_add: weight blob does not match the descriptor")
-    _require_numel(bn_scale, s.C_out, torch.float32, "bn_scale")
-    _require_numel(bn_bias, s.C_out, torch.float32, "bn_bias")
+    p = _plan(s)
+    _check_fused("fused_sparse_conv_bn_lif_add", s, p, data, values, meta, bn_scale, bn_bias,
+                 extra=((residual, "residual"),))
+    M, dev = p.M, data.device
     if f16 and residual_planes == 0:
         out_planes = 0
         _require_numel(residual, s.T * M * s.C_out, torch.float16, "residual")
     else:
         _require_numel(residual, s.T * M * residual_planes * s.C_out // 32, torch.int32, "residual")
-    if state is not None:
-        _require_cuda(state, "state")
-        _require_numel(state, M * s.C_out, torch.float32, "state")
+    _check_opt(state, M * s.C_out, torch.float32, "state")
     if out is None:
-        out = (torch.empty(s.T * s.B, OH, OW, s.C_out, dtype=torch.float16, device=dev) if f16 else
-               torch.empty(s.T * s.B, OH, OW, out_planes * s.C_out // 32, dtype=torch.int32, device=dev))
+        out = (torch.empty((s.T * s.B, p.OH, p.OW, s.C_out), dtype=torch.float16, device=dev) if f16 else
+               torch.empty((s.T * s.B, p.OH, p.OW, out_planes * s.C_out // 32), dtype=torch.int32, device=dev))
+    elif f16:
+        _check_opt(out, s.T * M * s.C_out, torch.float16, "out")
     else:
-        _require_cuda(out, "out")
-        if f16:
-            _require_numel(out, s.T * M * s.C_out, torch.float16, "out")
-        else:
-            _require_numel(out, s.T * M * out_planes * s.C_out // 32, torch.int32, "out")
-    rc = lib.sengine_amd_fused_sparse_conv_bn_lif_add(
-        ctypes.byref(d), _ptr(data), _ptr(values), _ptr(meta), _ptr(state), _ptr(bn_scale), _ptr(bn_bias),
-        _ptr(residual), int(residual_planes), _ptr(out), int(out_planes), _stream(dev))
-    check(rc, "fused_sparse_conv_bn_lif_add")
+        _check_opt(out, s.T * M * out_planes * s.C_out // 32, torch.int32, "out")
+    check(lib.sengine_amd_fused_sparse_conv_bn_lif_add(
+        p.ref, _ptr(data), _ptr(values), _ptr(meta), _ptr(state), _ptr(bn_scale), _ptr(bn_bias), _ptr(residual),
+        int(residual_planes), _ptr(out), int(out_planes), _stream(dev)), "fused_sparse_conv_bn_lif_add")
     return out
 
 
@@ -480,42 +561,24 @@ def fused_sparse_conv_bn_add_neuron(s: ConvSpec, data: torch.Tensor, values: tor
     """Membrane-shortcut form (MS-ResNet): y = BN(conv(data)) + residual (fp32 NHWC
     (T*B, OH, OW, C_out), or none) and the neuron of `s` run over y.  Returns (y, spikes)."""
     lib = _lib.load()
-    OH, OW, M, _ = geometry(s)
-    d = make_desc(s)
-    vb, mb = ctypes.c_size_t(), ctypes.c_size_t()
-    check(lib.sengine_amd_sparse_blob_bytes(ctypes.byref(d), ctypes.byref(vb), ctypes.byref(mb)), "sparse_blob_bytes")
-    for t, n in ((data, "data"), (values, "values"), (meta, "meta"), (bn_scale, "bn_scale"), (bn_bias, "bn_bias")):
-        _require_cuda(t, n)
+    p = _plan(s)
+    _check_fused("fused_sparse_conv_bn_add_neuron", s, p, data, values, meta, bn_scale, bn_bias)
     dev = data.device
-    dt, n_in = _enc_numel(s.in_enc, s.T * s.B * s.H * s.W * s.C_in)
-    _require_numel(data, n_in, dt, "data")
-    if values.numel() * values.element_size() != vb.value or meta.numel() * meta.element_size() != mb.value:
-        raise SEngineError("fused_sparse_conv_bn_add_neuron: weight blob does not match the descriptor")
-    _require_numel(bn_scale, s.C_out, torch.float32, "bn_scale")
-    _require_numel(bn_bias, s.C_out, torch.float32, "bn_bias")
-    n_real = s.T * M * s.C_out
-    if residual is not None:
-        _require_cuda(residual, "residual")
-        _require_numel(residual, n_real, torch.float32, "residual")
-    if state is not None:
-        _require_cuda(state, "state")
-        _require_numel(state, M * s.C_out, torch.float32, "state")
+    n_real = s.T * p.M * s.C_out
+    _check_opt(residual, n_real, torch.float32, "residual")
+    _check_opt(state, p.M * s.C_out, torch.float32, "state")
     if real_out is None:
-        real_out = torch.empty(s.T * s.B, OH, OW, s.C_out, dtype=torch.float32, device=dev)
+        real_out = torch.empty((s.T * s.B, p.OH, p.OW, s.C_out), dtype=torch.float32, device=dev)
     else:
-        _require_cuda(real_out, "real_out")
-        _require_numel(real_out, n_real, torch.float32, "real_out")
-    odt, n_out = _enc_numel(s.out_enc, s.T * M * s.C_out)
+        _check_opt(real_out, n_real, torch.float32, "real_out")
+    odt, n_out, shape = p.spikes(s)
     if out is None:
-        last = s.C_out // 32 if s.out_enc == ENC_BITS else s.C_out
-        out = torch.empty(s.T * s.B, OH, OW, last, dtype=odt, device=dev)
+        out = torch.empty(shape, dtype=odt, device=dev)
     else:
-        _require_cuda(out, "out")
-        _require_numel(out, n_out, odt, "out")
-    rc = lib.sengine_amd_fused_sparse_conv_bn_add_neuron(
-        ctypes.byref(d), _ptr(data), _ptr(values), _ptr(meta), _ptr(state), _ptr(bn_scale), _ptr(bn_bias),
-        _ptr(residual), _ptr(real_out), _ptr(out), _stream(dev))
-    check(rc, "fused_sparse_conv_bn_add_neuron")
+        _check_opt(out, n_out, odt, "out")
+    check(lib.sengine_amd_fused_sparse_conv_bn_add_neuron(
+        p.ref, _ptr(data), _ptr(values), _ptr(meta), _ptr(state), _ptr(bn_scale), _ptr(bn_bias), _ptr(residual),
+        _ptr(real_out), _ptr(out), _stream(dev)), "fused_sparse_conv_bn_add_neuron")
     return real_out, out
 
 
@@ -556,19 +619,16 @@ def spiking_self_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, T:
     lib = _lib.load()
     n_bits = T * B * N * C // 32
     for t, name in ((q, "q"), (k, "k"), (v, "v")):
-        _require_cuda(t, name)
-        _require_numel(t, n_bits, torch.int32, name)
+        _check_req(t, n_bits, torch.int32, name)
     d = C // heads if heads else 0
     if kv is None:
-        kv = torch.empty(T * B, heads, d, d, dtype=torch.int32, device=q.device)
+        kv = torch.empty((T * B, heads, d, d), dtype=torch.int32, device=q.device)
     else:
-        _require_cuda(kv, "kv")
-        _require_numel(kv, T * B * heads * d * d, torch.int32, "kv")
+        _check_req(kv, T * B * heads * d * d, torch.int32, "kv")
     if out is None:
-        out = torch.empty(T * B, N, C // 32, dtype=torch.int32, device=q.device)
+        out = torch.empty((T * B, N, C // 32), dtype=torch.int32, device=q.device)
     else:
-        _require_cuda(out, "out")
-        _require_numel(out, n_bits, torch.int32, "out")
+        _check_req(out, n_bits, torch.int32, "out")
     st = _stream(q.device)
     check(lib.sengine_amd_ssa_kv(T, B, N, C, heads, _ptr(k), _ptr(v), _ptr(kv), st), "ssa_kv")
     hard = v_reset is not None
@@ -644,28 +704,23 @@ def stem_conv_bn_neuron(s: ConvSpec, x: torch.Tensor, weight_hwio: torch.Tensor,
     (s.T*s.B, OH, OW, C_out/32), the layout of multistep_neuron_repeat on `out`), in one
     launch.  Returns (out or None, spikes)."""
     lib = _lib.load()
-    for t, n in ((x, "x"), (weight_hwio, "weight_hwio"), (bn_scale, "bn_scale"), (bn_bias, "bn_bias")):
-        _require_cuda(t, n)
-    _require_numel(x, s.B * s.C_in * s.H * s.W, torch.float32, "x")
-    _require_numel(weight_hwio, s.C_out * s.C_in * s.KH * s.KW, torch.float32, "weight_hwio")
-    _require_numel(bn_scale, s.C_out, torch.float32, "bn_scale")
-    _require_numel(bn_bias, s.C_out, torch.float32, "bn_bias")
+    _check_req(x, s.B * s.C_in * s.H * s.W, torch.float32, "x")
+    _check_req(weight_hwio, s.C_out * s.C_in * s.KH * s.KW, torch.float32, "weight_hwio")
+    _check_req(bn_scale, s.C_out, torch.float32, "bn_scale")
+    _check_req(bn_bias, s.C_out, torch.float32, "bn_bias")
     OH = (s.H + 2 * s.padding - s.KH) // s.stride + 1
     OW = (s.W + 2 * s.padding - s.KW) // s.stride + 1
     if out is None and want_out:
-        out = torch.empty(s.B, OH, OW, s.C_out, dtype=torch.float32, device=x.device)
-    elif out is not None:
-        _require_cuda(out, "out")
-        _require_numel(out, s.B * OH * OW * s.C_out, torch.float32, "out")
-    if spikes is None:
-        spikes = torch.empty(s.T * s.B, OH, OW, s.C_out // 32, dtype=torch.int32, device=x.device)
+        out = torch.empty((s.B, OH, OW, s.C_out), dtype=torch.float32, device=x.device)
     else:
-        _require_cuda(spikes, "spikes")
-        _require_numel(spikes, s.T * s.B * OH * OW * s.C_out // 32, torch.int32, "spikes")
-    d = make_desc(s)
-    check(lib.sengine_amd_stem_conv_bn_neuron(ctypes.byref(d), _ptr(x), _ptr(weight_hwio), _ptr(bn_scale),
-                                              _ptr(bn_bias), _ptr(out) if out is not None else None, _ptr(spikes),
-                                              _stream(x.device)), "stem_conv_bn_neuron")
+        _check_opt(out, s.B * OH * OW * s.C_out, torch.float32, "out")
+    if spikes is None:
+        spikes = torch.empty((s.T * s.B, OH, OW, s.C_out // 32), dtype=torch.int32, device=x.device)
+    else:
+        _check_req(spikes, s.T * s.B * OH * OW * s.C_out // 32, torch.int32, "spikes")
+    check(lib.sengine_amd_stem_conv_bn_neuron(_ref(s), x.data_ptr(), weight_hwio.data_ptr(), bn_scale.data_ptr(),
+                                              bn_bias.data_ptr(), _ptr(out), spikes.data_ptr(), _stream(x.device)),
+          "stem_conv_bn_neuron")
     return out, spikes
 
 
@@ -749,25 +804,21 @@ def dense_conv_bn(s: ConvSpec, data: torch.Tensor, values: torch.Tensor, bn_scal
                   bn_bias: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Dense Conv + folded BN -> fp32 (T*B, OH, OW, C_out)."""
     lib = _lib.load()
-    OH, OW, M, _ = geometry(s)
-    d = make_desc(s)
-    vb = ctypes.c_size_t()
-    check(lib.sengine_amd_dense_blob_bytes(ctypes.byref(d), ctypes.byref(vb)), "dense_blob_bytes")
-    for t, n in ((data, "data"), (values, "values"), (bn_scale, "bn_scale"), (bn_bias, "bn_bias")):
-        _require_cuda(t, n)
-    dt, n_in = _enc_numel(s.in_enc, s.T * s.B * s.H * s.W * s.C_in)
-    _require_numel(data, n_in, dt, "data")
-    if values.numel() * values.element_size() != vb.value:
+    p = _plan(s)
+    vb = p.dense_blob()
+    _require_cuda(values, "values")
+    dt, n_in = p.data(s)
+    _check_req(data, n_in, dt, "data")
+    if values.nbytes != vb:
         raise SEngineError("dense_conv_bn: weight blob does not match the descriptor")
-    _require_numel(bn_scale, s.C_out, torch.float32, "bn_scale")
-    _require_numel(bn_bias, s.C_out, torch.float32, "bn_bias")
+    _check_req(bn_scale, s.C_out, torch.float32, "bn_scale")
+    _check_req(bn_bias, s.C_out, torch.float32, "bn_bias")
     if out is None:
-        out = torch.empty(s.T * s.B, OH, OW, s.C_out, dtype=torch.float32, device=data.device)
+        out = torch.empty((s.T * s.B, p.OH, p.OW, s.C_out), dtype=torch.float32, device=data.device)
     else:
-        _require_cuda(out, "out")
-        _require_numel(out, s.T * M * s.C_out, torch.float32, "out")
-    check(lib.sengine_amd_dense_conv_bn(ctypes.byref(d), _ptr(data), _ptr(values), _ptr(bn_scale), _ptr(bn_bias),
-                                        _ptr(out), _stream(data.device)), "dense_conv_bn")
+        _check_opt(out, s.T * p.M * s.C_out, torch.float32, "out")
+    check(lib.sengine_amd_dense_conv_bn(p.ref, _ptr(data), _ptr(values), _ptr(bn_scale), _ptr(bn_bias), _ptr(out),
+                                        _stream(data.device)), "dense_conv_bn")
     return out
 
 
@@ -782,18 +833,13 @@ def multistep_neuron(x: torch.Tensor, T: int, neuron: str = "lif", tau: float = 
     if x.dtype != torch.float32 or x.numel() % T:
         raise SEngineError("multistep_neuron: x must be fp32 with T * n elements")
     n = x.numel() // T
-    if state is not None:
-        _require_cuda(state, "state")
-        _require_numel(state, n, torch.float32, "state")
-    if h_trace is not None:
-        _require_cuda(h_trace, "h_trace")
-        _require_numel(h_trace, T * n, torch.float32, "h_trace")
+    _check_opt(state, n, torch.float32, "state")
+    _check_opt(h_trace, T * n, torch.float32, "h_trace")
     odt, n_out = _enc_numel(out_enc, T * n)
     if out is None:
         out = torch.empty(n_out, dtype=odt, device=x.device)
     else:
-        _require_cuda(out, "out")
-        _require_numel(out, n_out, odt, "out")
+        _check_req(out, n_out, odt, "out")
     hard = v_reset is not None
     check(lib.sengine_amd_multistep_neuron(T, n, neuron_code(neuron), int(hard), float(tau),
                                            float(v_threshold), float(v_reset if hard else 0.0), _ptr(x), _ptr(state),

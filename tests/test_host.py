@@ -183,3 +183,23 @@ def test_compile_all_caches_kernels_by_shape():
     assert kern.spec.neuron == "lif" and kern.spec.tau == 2.0 and kern.spec.T == 4 and kern.spec.B == 2
     with pytest.raises(ops.SEngineError):
         SparseKernelCompiler(ir, batch_size=3).compile_all()  # T*B mismatch with the graph
+
+
+def test_spec_derived_state_stays_derived():
+    """What a ConvSpec keeps about itself (descriptor, plan, encoding variants) follows its fields
+    alone: equality, hash, replace, copies and pickles see only the fields."""
+    import copy
+    import dataclasses
+    import pickle
+
+    s = ops.ConvSpec(T=4, B=2, C_in=64, H=9, W=7, C_out=128, stride=2)
+    p = ops._plan(s)
+    assert ops._plan(s) is p and (p.OH, p.OW, p.M) == ops.geometry(s)[:3]
+    v = s.with_enc(ops.ENC_F16, ops.ENC_F16)
+    assert v is s.with_enc(ops.ENC_F16, ops.ENC_F16) and v == dataclasses.replace(s, in_enc=1, out_enc=1)
+    assert p.spikes(s) == (torch.int32, 4 * 2 * 5 * 4 * 4, (8, 5, 4, 4))
+    assert ops._plan(v).spikes(v) == (torch.float16, 4 * 2 * 5 * 4 * 128, (8, 5, 4, 128))
+    for c in (copy.copy(s), copy.deepcopy(s), pickle.loads(pickle.dumps(s)), dataclasses.replace(s)):
+        assert c == s and hash(c) == hash(s) and set(vars(c)) == {f.name for f in dataclasses.fields(s)}
+    wide = dataclasses.replace(s, C_out=192)
+    assert ops._plan(wide).spikes(wide)[2] == (8, 5, 4, 6) and ops._plan(wide).blob() != p.blob()
