@@ -306,6 +306,218 @@ __device__ __forceinline__ void smallm_body(const FusedParams& p, const int bx, 
                                  p.x_trace, p.sew, &res);
 }
 
+// ---- the same split for hard-reset neurons with spike-bit output, epilogue spread over all waves ----
+// The form above ends in one wave: it reads the whole sum back from LDS and runs 16 channels x T
+// steps per lane while the other seven wait, and its three operand sets move down by register
+// copies.  Here each of the 512 threads sums the eight partials of NA / 2 channels of one position,
+// runs BN and the neuron over T for them from those registers (membrane state included), and the
+// spike bits meet in LDS: thread (t, lane) then holds the 4 NA channels of a position and step,
+// adds the SEW residual and stores.  NA = 2 (a workgroup of 32 channels, byte stores) doubles the
+// workgroups where 64-channel ones leave CUs idle.  Operands are requested D - 1 chunks ahead in a
+// ring that is unrolled, not moved.  Same sums in the same order.
+//
+// Latency bound (a few chunks per wave): what counts is the chain launch -> operands -> sum ->
+// neuron -> store.  64->64 32x32 k3, one image, T = 4, two
+// weight planes: 11.2 -> 4.5 us; 512->512 7x7, four images: 13.8 -> 11.0 (two planes 22.8 -> 12.7);
+// SEW-ResNet-18 at 32x32, 64 images (16 such launches): 155 -> 132 us.
+template <int T, int PLANES, int NA>
+struct SpreadOperands {
+  half8_t av[PLANES][NA];
+  uint32_t ix[NA];
+  uint2 bw[T];
+};
+
+template <int T, int PLANES, int MODE, int NA>
+__device__ __forceinline__ void smallms_body(const FusedParams& p, const int bx, const int gy) {
+  constexpr int S = kSmallWaves;
+  constexpr int TR = T < 4 ? T : 4;        // timesteps per reduction round
+  constexpr int CPT = NA / 2;              // channels per thread of the epilogue (512 threads)
+  constexpr int HPT = 4 / CPT;             // threads per (tile, lane)
+  constexpr int D = NA == 2 ? (T * PLANES <= 4 ? 4 : 2) : (T * PLANES <= 4 ? 3 : 2);
+  const int G = NA == 4 ? gy : gy >> 1;
+  const int a0 = NA == 4 ? 0 : (gy & 1) * 2;  // first tile of the 64-channel group
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  const int g = lane >> 4;
+  const int col = lane & 15;
+  __shared__ float red[S][TR][NA * 256];
+  __shared__ uint16_t sbits[NA * 4 / CPT][64];
+
+  // everything the epilogue reads from memory is requested now, next to the first operands
+  // its thread: float f = tid * CPT of a (tile, lane, channel-of-four) row of sums
+  const int el = (tid * CPT / 4) & 63, ea = tid * CPT / 256, er = (tid * CPT) & 3;
+  const int em = bx * 16 + (el & 15);                       // position
+  const int ec = G * 64 + 16 * (el >> 4) + 4 * (a0 + ea) + er;  // first channel
+  const bool evalid = em < p.M;
+  float sc[CPT], bi[CPT], v[CPT];
+#pragma unroll
+  for (int i = 0; i < CPT; ++i) {
+    const int c = (G * 64) % p.bn_period + ec - G * 64 + i;
+    sc[i] = p.scale[c];
+    bi[i] = p.bias[c];
+    v[i] = p.state && evalid ? p.state[(size_t)em * p.F + ec + i] : 0.f;
+  }
+  // the storing thread: step st (one wave per step), position sm, channels sch .. sch + 4 NA - 1
+  const int st = wave;
+  const int sm = bx * 16 + col;
+  const int sch = G * 64 + 16 * g + 4 * a0;
+  const bool storing = st < T && sm < p.M;
+  const int spix = sch / p.sew.pix_ch, sc0 = sch - spix * p.sew.pix_ch;
+  uint32_t rp[kMaxPlanes] = {};
+  if (storing && p.sew.res) {
+    const size_t rbase =
+        ((size_t)st * p.M + sm) * p.sew.res_planes * p.F + (size_t)spix * p.sew.res_planes * p.sew.pix_ch + sc0;
+#pragma unroll
+    for (int pl = 0; pl < kMaxPlanes; ++pl)
+      if (pl < p.sew.res_planes) {
+        const uint8_t* r = p.sew.res + ((rbase + (size_t)pl * p.sew.pix_ch) >> 3);
+        rp[pl] = NA == 4 ? (uint32_t)*reinterpret_cast<const uint16_t*>(r) : (uint32_t)*r;
+      }
+  }
+
+  float4_t acc[T][NA];
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int a = 0; a < NA; ++a) acc[t][a] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+  const int nq = p.nq;
+  const int m = bx * 16 + col;
+  const bool mvalid = m < p.M;
+  int b = 0, oh = 0, ow = 0;
+  if (mvalid) {
+    const int ohw = p.OH * p.OW;
+    b = m / ohw;
+    const int r = m - b * ohw;
+    oh = r / p.OW;
+    ow = r - oh * p.OW;
+  }
+  const int cbytes = p.C >> 3;
+  const int chunks_per_tap = p.C >> 6;
+  const size_t tstride = (size_t)p.in_t_stride * cbytes;
+  const half8_t* wv = p.wvals + (size_t)G * nq * PLANES * 4 * 64 + a0 * 64 + lane;
+  const uint32_t* wm = p.wmeta + (size_t)G * nq * 4 * 64 + lane * 4 + a0;  // [q][lane][tile]
+  const uint32_t sel = 0x0c0c0000u | ((uint32_t)(4 + g) << 8) | (uint32_t)g;
+
+  auto load = [&](int q, SpreadOperands<T, PLANES, NA>& o) {
+#pragma unroll
+    for (int a = 0; a < NA; ++a) {
+#pragma unroll
+      for (int pl = 0; pl < PLANES; ++pl) o.av[pl][a] = wv[((size_t)(q * PLANES + pl) * 4 + a) * 64];
+    }
+    typedef uint32_t ix_t __attribute__((ext_vector_type(NA)));
+    const ix_t mx = *reinterpret_cast<const ix_t*>(wm + (size_t)q * 4 * 64);
+#pragma unroll
+    for (int a = 0; a < NA; ++a) o.ix[a] = mx[a];
+    const int tap = q / chunks_per_tap;
+    const int c0 = q - tap * chunks_per_tap;
+    const int kr = tap / p.KW;
+    const int ih = oh * p.SH - p.PH + kr * p.DH;
+    const int iw = ow * p.SW - p.PW + (tap - kr * p.KW) * p.DW;
+    const bool ok = mvalid && ih >= 0 && ih < p.H && iw >= 0 && iw < p.W;
+    const uint8_t* src = p.in + (((size_t)b * p.H + (ok ? ih : 0)) * p.W + (ok ? iw : 0)) * cbytes + c0 * 8;
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+      o.bw[t] = ok ? *reinterpret_cast<const uint2*>(src + t * tstride) : uint2{0u, 0u};
+  };
+  SpreadOperands<T, PLANES, NA> o[D];
+#pragma unroll
+  for (int u = 0; u < D - 1; ++u)
+    if (wave + u * S < nq) load(wave + u * S, o[u]);
+  for (int q0 = wave; q0 < nq; q0 += D * S) {
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+      const int q = q0 + u * S;
+      if (q >= nq) break;
+      if (q + (D - 1) * S < nq) load(q + (D - 1) * S, o[(u + D - 1) % D]);
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        const half16_t bf = expand_bits16(__builtin_amdgcn_perm(o[u].bw[t].y, o[u].bw[t].x, sel));
+#pragma unroll
+        for (int a = 0; a < NA; ++a)
+#pragma unroll
+          for (int pl = 0; pl < PLANES; ++pl)
+            acc[t][a] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(o[u].av[pl][a], bf, acc[t][a], o[u].ix[a], 0, 0);
+      }
+    }
+  }
+
+#pragma unroll
+  for (int i = 0; i < CPT; ++i) {
+    sc[i] *= p.enc_scale;
+    if (MODE == EPI_LIF_HARD) {
+      sc[i] *= p.np.rtau;  // exact: a power of two
+      bi[i] *= p.np.rtau;
+    }
+  }
+  uint32_t bits = 0;
+#pragma unroll
+  for (int t0 = 0; t0 < T; t0 += TR) {
+    if (t0) __syncthreads();
+#pragma unroll
+    for (int u = 0; u < TR; ++u)
+#pragma unroll
+      for (int a = 0; a < NA; ++a) *reinterpret_cast<float4_t*>(&red[wave][u][a * 256 + lane * 4]) = acc[t0 + u][a];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < TR; ++u) {
+      float sum[CPT];
+#pragma unroll
+      for (int w = 0; w < S; ++w)  // in wave order
+#pragma unroll
+        for (int i = 0; i < CPT; ++i) {
+          const float x = red[w][u][tid * CPT + i];
+          sum[i] = w == 0 ? x : sum[i] + x;
+        }
+#pragma unroll
+      for (int i = 0; i < CPT; ++i) {
+        const float xin = __builtin_fmaf(sum[i], sc[i], bi[i]);
+        const float h = MODE == EPI_LIF_HARD ? __builtin_fmaf(v[i], p.np.decay, xin) : __fadd_rn(v[i], xin);
+        const bool spike = h >= p.np.vth;
+        v[i] = spike ? p.np.vreset : h;
+        bits |= (uint32_t)spike << ((t0 + u) * CPT + i);
+      }
+    }
+  }
+  if (p.state && evalid) {
+#pragma unroll
+    for (int i = 0; i < CPT; ++i) p.state[(size_t)em * p.F + ec + i] = v[i];
+  }
+  sbits[ea * HPT + er / CPT][el] = (uint16_t)bits;
+  __syncthreads();
+  if (!storing) return;
+  uint32_t word = 0;
+#pragma unroll
+  for (int i = 0; i < NA * HPT; ++i)
+    word |= (((uint32_t)sbits[i][lane] >> (st * CPT)) & ((1u << CPT) - 1u)) << (i * CPT);
+  auto put = [&](uint8_t* dst, uint32_t w) {
+    if (NA == 4)
+      *reinterpret_cast<uint16_t*>(dst) = (uint16_t)w;
+    else
+      *dst = (uint8_t)w;
+  };
+  const size_t row = (size_t)st * p.M + sm;
+  if (p.sew.res == nullptr) {
+    const SpikeDst sd = spike_dst(p.sew, p.out, p.F, sch);
+    put(sd.out + ((row * sd.F + sd.cob) >> 3), word);
+    return;
+  }
+  const size_t obase = row * (size_t)p.sew.out_planes * p.F + (size_t)spix * p.sew.out_planes * p.sew.pix_ch + sc0;
+  uint32_t carry = word;
+#pragma unroll
+  for (int pl = 0; pl < kMaxPlanes; ++pl) {
+    if (pl >= p.sew.out_planes) break;
+    put(p.out + ((obase + (size_t)pl * p.sew.pix_ch) >> 3), rp[pl] ^ carry);
+    carry &= rp[pl];
+  }
+}
+
+template <int T, int PLANES, int MODE, int NA>
+__global__ __launch_bounds__(64 * kSmallWaves) void fused_smallms_kernel(FusedParams p) {
+  smallms_body<T, PLANES, MODE, NA>(p, (int)blockIdx.x, (int)blockIdx.y);
+}
+
 template <int T, int OUT_ENC, int PLANES, int MODE>
 __global__ __launch_bounds__(64 * kSmallWaves) void fused_smallm_kernel(FusedParams p) {
   smallm_body<T, OUT_ENC, PLANES, MODE>(p, (int)blockIdx.x, (int)blockIdx.y);
@@ -322,21 +534,51 @@ __global__ __launch_bounds__(64 * kSmallWaves) void fused_smallm_pair_kernel(Fus
   smallm_body<T, OUT_ENC, PLANES, MODE>(p, (int)blockIdx.x, second ? (int)blockIdx.y - g0 : (int)blockIdx.y);
 }
 
+template <int T, int PLANES, int MODE, int NA>
+__global__ __launch_bounds__(64 * kSmallWaves) void fused_smallms_pair_kernel(FusedParams p0, FusedParams p1, int g0) {
+  const bool second = (int)blockIdx.y >= g0;
+  const FusedParams& p = second ? p1 : p0;
+  if ((int)blockIdx.x * 16 >= p.M) return;
+  smallms_body<T, PLANES, MODE, NA>(p, (int)blockIdx.x, second ? (int)blockIdx.y - g0 : (int)blockIdx.y);
+}
+
+// 64-channel workgroups of the spread form below this many (one per CU) become pairs of 32-channel
+// ones: 64 workgroups (64->64 32x32, one image, two weight planes) 5.4 -> 4.5 us, 104 (512->512
+// 7x7, four images) 12.3 -> 11.0; but 256 (64->64 8x8, 64 images) 5.3 -> 7.2, since a pair expands
+// the same spikes twice.
+constexpr int64_t kSmallSplitBelow = 256;
+
 template <int T>
 static hipError_t launch_smallm(const FusedParams& p, int out_enc, int planes, int mode, hipStream_t s) {
   const dim3 grid((unsigned)((p.M + 15) / 16), (unsigned)(p.F / 64));
   const dim3 block(64 * kSmallWaves);
-#define SENGINE_SMALLM_CASE(OE, PL, MD)                  \
-  if (out_enc == OE && planes == PL && mode == MD) {     \
-    hipLaunchKernelGGL((fused_smallm_kernel<T, OE, PL, MD>), grid, block, 0, s, p); \
+  if (mode != EPI_GENERIC) {  // spike-bit output (plan_fused)
+    const bool split = (int64_t)grid.x * grid.y < kSmallSplitBelow;
+    const dim3 grid2(grid.x, grid.y * 2);
+#define SENGINE_SMALLMS_CASE(PL, MD)                                                             \
+  if (planes == PL && mode == MD) {                                                              \
+    if (split)                                                                                   \
+      hipLaunchKernelGGL((fused_smallms_kernel<T, PL, MD, 2>), grid2, block, 0, s, p);           \
+    else                                                                                         \
+      hipLaunchKernelGGL((fused_smallms_kernel<T, PL, MD, 4>), grid, block, 0, s, p);            \
+    return hipGetLastError();                                                                    \
+  }
+    SENGINE_SMALLMS_CASE(1, EPI_LIF_HARD)
+    SENGINE_SMALLMS_CASE(1, EPI_IF_HARD)
+    SENGINE_SMALLMS_CASE(2, EPI_LIF_HARD)
+    SENGINE_SMALLMS_CASE(2, EPI_IF_HARD)
+#undef SENGINE_SMALLMS_CASE
+    return hipErrorInvalidValue;
+  }
+#define SENGINE_SMALLM_CASE(OE, PL)                      \
+  if (out_enc == OE && planes == PL) {                   \
+    hipLaunchKernelGGL((fused_smallm_kernel<T, OE, PL, EPI_GENERIC>), grid, block, 0, s, p); \
     return hipGetLastError();                            \
   }
-  SENGINE_SMALLM_CASE(SENGINE_ENC_BITS, 1, EPI_LIF_HARD)
-  SENGINE_SMALLM_CASE(SENGINE_ENC_BITS, 1, EPI_IF_HARD)
-  SENGINE_SMALLM_CASE(SENGINE_ENC_BITS, 1, EPI_GENERIC)
-  SENGINE_SMALLM_CASE(SENGINE_ENC_BITS, 2, EPI_GENERIC)
-  SENGINE_SMALLM_CASE(SENGINE_ENC_F16, 1, EPI_GENERIC)
-  SENGINE_SMALLM_CASE(SENGINE_ENC_F16, 2, EPI_GENERIC)
+  SENGINE_SMALLM_CASE(SENGINE_ENC_BITS, 1)
+  SENGINE_SMALLM_CASE(SENGINE_ENC_BITS, 2)
+  SENGINE_SMALLM_CASE(SENGINE_ENC_F16, 1)
+  SENGINE_SMALLM_CASE(SENGINE_ENC_F16, 2)
 #undef SENGINE_SMALLM_CASE
   return hipErrorInvalidValue;
 }
@@ -347,15 +589,32 @@ static hipError_t launch_smallm_pair(const FusedParams& p0, const FusedParams& p
   const int g0 = p0.F / 64;
   const dim3 grid((unsigned)((std::max(p0.M, p1.M) + 15) / 16), (unsigned)(g0 + p1.F / 64));
   const dim3 block(64 * kSmallWaves);
-#define SENGINE_SMALLM_PAIR_CASE(OE, PL, MD)                                        \
-  if (out_enc == OE && planes == PL && mode == MD) {                               \
-    hipLaunchKernelGGL((fused_smallm_pair_kernel<T, OE, PL, MD>), grid, block, 0, s, p0, p1, g0); \
-    return hipGetLastError();                                                      \
+  if (mode != EPI_GENERIC) {
+    const bool split = (int64_t)grid.x * grid.y < kSmallSplitBelow;
+    const dim3 grid2(grid.x, grid.y * 2);
+#define SENGINE_SMALLMS_PAIR_CASE(PL, MD)                                                                   \
+  if (planes == PL && mode == MD) {                                                                         \
+    if (split)                                                                                              \
+      hipLaunchKernelGGL((fused_smallms_pair_kernel<T, PL, MD, 2>), grid2, block, 0, s, p0, p1, g0 * 2);    \
+    else                                                                                                    \
+      hipLaunchKernelGGL((fused_smallms_pair_kernel<T, PL, MD, 4>), grid, block, 0, s, p0, p1, g0);         \
+    return hipGetLastError();                                                                               \
   }
-  SENGINE_SMALLM_PAIR_CASE(SENGINE_ENC_BITS, 1, EPI_LIF_HARD)
-  SENGINE_SMALLM_PAIR_CASE(SENGINE_ENC_BITS, 1, EPI_IF_HARD)
-  SENGINE_SMALLM_PAIR_CASE(SENGINE_ENC_BITS, 1, EPI_GENERIC)
-  SENGINE_SMALLM_PAIR_CASE(SENGINE_ENC_BITS, 2, EPI_GENERIC)
+    SENGINE_SMALLMS_PAIR_CASE(1, EPI_LIF_HARD)
+    SENGINE_SMALLMS_PAIR_CASE(1, EPI_IF_HARD)
+    SENGINE_SMALLMS_PAIR_CASE(2, EPI_LIF_HARD)
+    SENGINE_SMALLMS_PAIR_CASE(2, EPI_IF_HARD)
+#undef SENGINE_SMALLMS_PAIR_CASE
+    return hipErrorInvalidValue;
+  }
+#define SENGINE_SMALLM_PAIR_CASE(PL)                                                \
+  if (out_enc == SENGINE_ENC_BITS && planes == PL) {                                \
+    hipLaunchKernelGGL((fused_smallm_pair_kernel<T, SENGINE_ENC_BITS, PL, EPI_GENERIC>), grid, block, 0, s, p0, p1, \
+                       g0);                                                         \
+    return hipGetLastError();                                                       \
+  }
+  SENGINE_SMALLM_PAIR_CASE(1)
+  SENGINE_SMALLM_PAIR_CASE(2)
 #undef SENGINE_SMALLM_PAIR_CASE
   return hipErrorInvalidValue;
 }
@@ -472,9 +731,9 @@ static int plan_fused(const sengine_conv_lif_desc* d, const void* data, const vo
   }
   if ((flat || small) && d->in_enc == SENGINE_ENC_BITS && choice != 1) {
     plan.route = kRouteSmall;
-    // fast epilogue modes for the common case (one weight plane, bit output)
+    // hard-reset neurons with bit output take the spread form (its modes compute what the generic one does)
     plan.mode = epilogue_mode(p.np, h_trace != nullptr || x_trace != nullptr || sew.real_out != nullptr);
-    if (d->weight_planes != 1 || d->out_enc != SENGINE_ENC_BITS) plan.mode = EPI_GENERIC;
+    if (d->out_enc != SENGINE_ENC_BITS) plan.mode = EPI_GENERIC;
   } else {
     plan.route = kRouteDirect;
   }
