@@ -301,6 +301,18 @@ int sengine_amd_ssa_attend_neuron(int32_t T, int32_t B, int32_t N, int32_t C, in
                                   const uint32_t* q_bits, const int32_t* kv, uint32_t* out_bits, hipStream_t stream);
 
 /*
+ * Both steps in one call: one launch that keeps K^T V in LDS, or the two entries above with kv between
+ * them.  sengine_amd_ssa_attention_needs_kv: 0 where a call is one launch -- with `workspace` nonzero,
+ * for a call that passes a kv (which receives K^T V all the same), else for one that passes null.
+ * Accepts what the two entries accept; the same bits.
+ */
+int sengine_amd_ssa_attention_needs_kv(int32_t T, int32_t B, int32_t N, int32_t C, int32_t heads, int32_t workspace);
+int sengine_amd_ssa_attention(int32_t T, int32_t B, int32_t N, int32_t C, int32_t heads, float scale,
+                              int32_t neuron, int32_t hard_reset, float tau, float v_threshold, float v_reset,
+                              const uint32_t* q_bits, const uint32_t* k_bits, const uint32_t* v_bits, int32_t* kv,
+                              uint32_t* out_bits, hipStream_t stream);
+
+/*
  * Allocation-free spiking self-attention: sengine_amd_ssa_kv followed by
  * sengine_amd_ssa_attend_neuron with the K^T V partial sums in a library-owned device array
  * instead of a caller workspace.  No counterpart in the reference: for callers that cannot

@@ -206,6 +206,11 @@ class SpikingSelfAttentionKernel:
         d = self.C // self.heads
         return self.T * self.B * self.heads * d * d
 
+    @property
+    def needs_kv(self) -> bool:
+        """Whether a call with a workspace is two launches around it (else one, and it needs none)."""
+        return ops.attention_needs_kv(self.T, self.B, self.N, self.C, self.heads, workspace=True)
+
     def __call__(self, q, k, v, kv=None, out=None):
         return ops.spiking_self_attention(q, k, v, self.T, self.B, self.N, self.C, self.heads, scale=self.scale,
                                           neuron="lif", tau=self.tau, v_threshold=self.v_threshold, v_reset=0.0,

@@ -399,6 +399,217 @@ __global__ __launch_bounds__(256) void ssa_attend_kernel(SsaParams p, int splits
   }
 }
 
+// Both halves in one workgroup per (b, head): K^T V stays in LDS, so nothing of it goes through
+// memory (T * d^2 * 4 bytes per (b, head) written and read back several times over by the two
+// kernels above) and one launch does.
+//
+//   K^T V: wave w takes timestep w % T and every (NW / T)-th 64-token group: lane n loads token n's
+//   head slices of K and V (the next group's are in flight), two butterfly transposes turn them into
+//   channel masks, and lane i adds popcount(K_i & V_j) for every j to registers, the V masks read
+//   back as LDS broadcasts.  The waves of a timestep meet in LDS by integer atomics (exact).
+//   Q (K^T V): the sums become fp16 pieces in LDS as in ssa_attend_kernel, and each wave walks
+//   16-token tiles: the products of all T steps first (exact in any order), then the neuron with its
+//   spikes shifted into nibbles; a 4 x 4 nibble transpose among the four lanes of a token gives each
+//   of them the channel words of one timestep, one store for four steps.
+//
+// Bound by VALU work (transposes, popcounts, the neuron); a (b, head) has little of it, so the launch
+// and the phases' latencies count at small N.  32 images, 8 heads of 48, T = 4: 196 tokens
+// 39.5 -> 14.6 us, 3,136 tokens 135.5 -> 92.4 us (both kernels before).
+template <int D, int T, int NW, bool FASTN>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) void ssa_fused_kernel(SsaParams p) {
+  constexpr int JT = D / 16;
+  constexpr int KS = (D + 31) / 32;
+  constexpr int RV = kSsaRow / 8;
+  constexpr int NT = 64 * NW;
+  constexpr int NSUB = NW / T;     // waves of one timestep
+  constexpr int SD = D + 1;        // row of sums: lanes i of a column fall on different banks
+  constexpr int PIECES = T * 2 * D * kSsaRow * 2;  // bytes
+  static_assert(NW % T == 0 && T * D * SD * 4 <= PIECES, "the sums fit under the pieces");
+  __shared__ __align__(16) uint8_t smem[PIECES];
+  __shared__ __align__(16) uint64_t sV[NW][D];
+  uint32_t* sum = reinterpret_cast<uint32_t*>(smem);      // [t][i][j], rows of SD
+  _Float16* s = reinterpret_cast<_Float16*>(smem);        // [t][piece][j][kSsaRow], after the sums
+  const half8_t* skv = reinterpret_cast<const half8_t*>(smem);
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int q = lane >> 4;
+  const int c = lane & 15;
+  // consecutive workgroup ids go round-robin over the XCDs: give each XCD a contiguous run, so the
+  // heads of an image, which share the lines of its token rows, share an L2
+  const int nwg = (int)gridDim.x, run = nwg >> 3;
+  const int id = (int)blockIdx.x;
+  const int bh = id < run * 8 ? (id & 7) * run + (id >> 3) : id;
+  const int b = bh / p.H;
+  const int h = bh - b * p.H;
+  const int words = p.C >> 5;
+
+  for (int i = tid; i < T * D * SD; i += NT) sum[i] = 0u;
+  __syncthreads();
+  {
+    const int t = wave % T;
+    const int G = (p.N + 63) >> 6;
+    const size_t row0 = (size_t)(t * p.B + b) * p.N;
+    auto load = [&](int g, uint64_t& kw, uint64_t& vw) {
+      const int n = (g << 6) + lane;
+      const bool in = g < G && n < p.N;
+      const size_t off = (row0 + (in ? n : 0)) * words;
+      kw = in ? head_slice(p.k + off, words, h * D, D) : 0ull;
+      vw = in ? head_slice(p.v + off, words, h * D, D) : 0ull;
+    };
+    uint32_t cnt[D];
+#pragma unroll
+    for (int j = 0; j < D; ++j) cnt[j] = 0u;
+    uint64_t kn, vn;
+    int g = wave / T;
+    load(g, kn, vn);
+    for (; g < G; g += NSUB) {
+      const uint64_t km = transpose64(kn, lane), vm = transpose64(vn, lane);
+      load(g + NSUB, kn, vn);
+      if (lane < D) sV[wave][lane] = vm;
+      __builtin_amdgcn_wave_barrier();  // one wave's LDS operations complete in order
+      const uint32_t klo = (uint32_t)km, khi = (uint32_t)(km >> 32);
+#pragma unroll
+      for (int j = 0; j < D; j += 2) {
+        const u32x4_t v2 = *reinterpret_cast<const u32x4_t*>(&sV[wave][j]);  // broadcast
+        cnt[j] += (uint32_t)__popc(klo & v2[0]) + (uint32_t)__popc(khi & v2[1]);
+        cnt[j + 1] += (uint32_t)__popc(klo & v2[2]) + (uint32_t)__popc(khi & v2[3]);
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+    if (lane < D) {
+#pragma unroll
+      for (int j = 0; j < D; ++j) atomicAdd(&sum[(t * D + lane) * SD + j], cnt[j]);
+    }
+  }
+  __syncthreads();
+  if (p.kv) {  // the caller's copy of K^T V
+    for (int e = tid; e < T * D * D; e += NT) {
+      const int t = e / (D * D), ij = e - t * (D * D);
+      p.kv[((size_t)(t * p.B + b) * p.H + h) * D * D + ij] = (int32_t)sum[(t * D + ij / D) * SD + ij % D];
+    }
+  }
+  // sums -> scaled fp16 pieces, transposed to [j][i]: through registers, the two share their LDS
+  constexpr int EPT = (T * D * D + NT - 1) / NT;
+  uint32_t x[EPT];
+#pragma unroll
+  for (int k = 0; k < EPT; ++k) {
+    const int e = tid + k * NT;
+    const int tj = e / D, i = e - tj * D, t = tj / D, j = tj - t * D;
+    x[k] = e < T * D * D ? sum[(t * D + i) * SD + j] : 0u;
+  }
+  __syncthreads();
+  int high = 0;
+#pragma unroll
+  for (int k = 0; k < EPT; ++k) {
+    const int e = tid + k * NT;
+    const int tj = e / D, i = e - tj * D, t = tj / D, j = tj - t * D;
+    if (e < T * D * D) {
+      s[((size_t)(t * 2 + 0) * D + j) * kSsaRow + i] = (_Float16)((float)(x[k] & 2047u) * p.xscale);
+      s[((size_t)(t * 2 + 1) * D + j) * kSsaRow + i] = (_Float16)((float)(x[k] & ~2047u) * p.xscale);
+      high |= (int)(x[k] & ~2047u);
+    }
+  }
+  if (D < 32 * KS) {  // rows i = D .. of the last k step read as zero
+    constexpr int PADI = 32 * KS - D > 0 ? 32 * KS - D : 1;
+    for (int e = tid; e < T * 2 * D * PADI; e += NT) {
+      const int row = e / PADI;
+      s[(size_t)row * kSsaRow + D + (e - row * PADI)] = (_Float16)0.f;
+    }
+  }
+  const bool big = __syncthreads_or(high != 0);  // some high piece is nonzero (workgroup-uniform)
+
+  const bool fold = p.np.neuron == SENGINE_NEURON_LIF && p.np.pow2;
+  const int tiles = (p.N + 15) >> 4;
+  const size_t in_t = (size_t)p.B * p.N * words;
+  auto load_q = [&](int tile, uint64_t (&qs)[T]) {
+    const int n = min(tile * 16 + c, p.N - 1);  // past the end: the last token, computed but not stored
+    const uint32_t* src = p.q + ((size_t)b * p.N + n) * words;
+#pragma unroll
+    for (int t = 0; t < T; ++t) qs[t] = head_slice(src + t * in_t, words, h * D, D);
+  };
+  uint64_t qn[T];
+  if (wave < tiles) load_q(wave, qn);
+  for (int tile = wave; tile < tiles; tile += NW) {
+    uint64_t qc[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) qc[t] = qn[t];
+    load_q(min(tile + NW, tiles - 1), qn);
+    const int n = tile * 16 + c;
+    float v[JT][4];
+#pragma unroll
+    for (int jt = 0; jt < JT; ++jt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[jt][e] = 0.f;
+#pragma unroll
+    for (int t0 = 0; t0 < T; t0 += 4) {
+      constexpr int TC = T < 4 ? T : 4;
+      uint32_t nib[JT];
+#pragma unroll
+      for (int jt = 0; jt < JT; ++jt) nib[jt] = 0u;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (k >= TC) {  // no such step: keep the steps' places
+#pragma unroll
+          for (int jt = 0; jt < JT; ++jt) nib[jt] <<= 4;
+          continue;
+        }
+        const int t = t0 + k;
+        const half8_t* st = skv + (size_t)t * 2 * D * RV;
+        float4_t acc[JT];
+#pragma unroll
+        for (int jt = 0; jt < JT; ++jt) acc[jt] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          const half8_t bq = expand_bits8((uint32_t)(qc[t] >> (32 * ks + 8 * q)) & 0xffu);
+#pragma unroll
+          for (int jt = 0; jt < JT; ++jt) {
+            acc[jt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(st[(size_t)(jt * 16 + c) * RV + ks * 4 + q], bq, acc[jt],
+                                                             0, 0, 0);
+            if (big)
+              acc[jt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(st[(size_t)(D + jt * 16 + c) * RV + ks * 4 + q], bq,
+                                                               acc[jt], 0, 0, 0);
+          }
+        }
+        // neuron on x[token][j = 16 jt + 4 q + e], spikes shifted in so that e = 0 ends lowest
+#pragma unroll
+        for (int jt = 0; jt < JT; ++jt)
+#pragma unroll
+          for (int e = 3; e >= 0; --e) {
+            const float xv = acc[jt][e];
+            if (FASTN) {
+              const float hh = __builtin_fmaf(v[jt][e], p.np.decay, xv);  // v*decay exact: one rounding
+              fire_hard(hh, p.np.vth, p.np.vreset, v[jt][e], nib[jt]);
+            } else {
+              const float hh = neuron_charge(p.np, v[jt][e], fold ? xv * p.np.rtau : xv);
+              const bool spike = hh >= p.np.vth;
+              v[jt][e] = neuron_reset(p.np, hh, spike);
+              nib[jt] = 2 * nib[jt] + (uint32_t)spike;
+            }
+          }
+      }
+      // nib: step t0 + k in nibble 3 - k; lane group q ends with the words of step t0 + 3 - q
+      const int t = t0 + 3 - q;
+      const bool st = n < p.N && 3 - q < TC;
+      uint16_t* o = p.out + (((size_t)t * p.B + b) * p.N + n) * (p.C / 16) + h * JT;
+#pragma unroll
+      for (int jt = 0; jt < JT; jt += 2) {
+        const uint32_t xw = nib[jt] | (jt + 1 < JT ? nib[jt + 1 < JT ? jt + 1 : 0] << 16 : 0u);
+        const uint32_t px = (uint32_t)__shfl_xor((int)xw, 32, 64);
+        const uint32_t y = q < 2 ? (xw & 0x00ff00ffu) | ((px & 0x00ff00ffu) << 8)
+                                 : (xw & 0xff00ff00u) | ((px & 0xff00ff00u) >> 8);
+        const uint32_t py = (uint32_t)__shfl_xor((int)y, 16, 64);
+        const uint32_t w = (q & 1) == 0 ? (y & 0x0f0f0f0fu) | ((py & 0x0f0f0f0fu) << 4)
+                                        : (y & 0xf0f0f0f0u) | ((py & 0xf0f0f0f0u) >> 4);
+        if (st) {
+          o[jt] = (uint16_t)w;
+          if (jt + 1 < JT) o[jt + 1] = (uint16_t)(w >> 16);
+        }
+      }
+    }
+  }
+}
+
 template <int D, int T>
 static void* attend_fn_t(bool fast) {
   return fast ? reinterpret_cast<void*>(&ssa_attend_kernel<D, T, EPI_LIF_HARD>)
@@ -521,6 +732,54 @@ int attend_launch(AttendLaunch& L, hipStream_t stream) {
   return (int)hipLaunchKernel(L.fn, dim3((unsigned)(L.p.B * L.p.H * L.splits)), dim3(256), args, L.lds, stream);
 }
 
+// Whether the one-workgroup-per-(b, head) kernel takes a call: long token grids of few (b, head)
+// pairs stay with the two kernels, which split the tokens over the chip.  Measured (T = 4, C = 384, 8
+// heads, two kernels / fused, us): 196 tokens, 8 pairs 19.6 / 13.6, 256 pairs 39.5 / 14.6; 784 tokens
+// (C = 512), 64 pairs 44.6 / 37.6; 3,136 tokens, 8 pairs 59.6 / 85.9, 64 pairs 82.8 / 86.8, 128 pairs
+// 97.6 / 88.7, 256 pairs 135.5 / 92.4.
+// A caller that brings a workspace (an engine plans its launches with it) gets the two kernels for
+// few pairs at any token count.
+bool fused_takes(int T, int B, int N, int heads, bool workspace) {
+  if (T != 1 && T != 2 && T != 4 && T != 8) return false;
+  return (N <= 768 && !workspace) || (int64_t)B * heads >= 96;
+}
+
+template <int D, int T>
+int fused_launch_dt(const SsaParams& p, bool fast, hipStream_t stream) {
+  const int64_t wgs = (int64_t)p.B * p.H;
+  constexpr bool WIDE_FITS = (size_t)T * 2 * D * kSsaRow * 2 + (size_t)16 * D * 8 <= kSsaMaxLds;
+  static_assert(WIDE_FITS, "every supported shape fits with sixteen waves");
+  // sixteen waves while a CU gets one workgroup, eight (two workgroups per CU) beyond
+  const dim3 grid((unsigned)wgs);
+  if (wgs <= 256 || T * D > 256) {
+    if (fast) hipLaunchKernelGGL((ssa_fused_kernel<D, T, 16, true>), grid, dim3(1024), 0, stream, p);
+    else hipLaunchKernelGGL((ssa_fused_kernel<D, T, 16, false>), grid, dim3(1024), 0, stream, p);
+  } else {
+    if (fast) hipLaunchKernelGGL((ssa_fused_kernel<D, T, 8, true>), grid, dim3(512), 0, stream, p);
+    else hipLaunchKernelGGL((ssa_fused_kernel<D, T, 8, false>), grid, dim3(512), 0, stream, p);
+  }
+  return (int)hipGetLastError();
+}
+
+template <int D>
+int fused_launch_d(const SsaParams& p, bool fast, hipStream_t stream) {
+  switch (p.T) {
+    case 1: return fused_launch_dt<D, 1>(p, fast, stream);
+    case 2: return fused_launch_dt<D, 2>(p, fast, stream);
+    case 4: return fused_launch_dt<D, 4>(p, fast, stream);
+    default: return fused_launch_dt<D, 8>(p, fast, stream);
+  }
+}
+
+int fused_launch(const SsaParams& p, bool fast, hipStream_t stream) {
+  switch (p.d) {
+    case 16: return fused_launch_d<16>(p, fast, stream);
+    case 32: return fused_launch_d<32>(p, fast, stream);
+    case 48: return fused_launch_d<48>(p, fast, stream);
+    default: return fused_launch_d<64>(p, fast, stream);
+  }
+}
+
 // Allocation-free attention: K^T V in a file-scope device array instead of a caller workspace.
 // Each GPU holds its own copy; its address is taken once per device (host code never passes
 // the array's name itself, which on the host is only a stand-in for the symbol).
@@ -590,5 +849,37 @@ extern "C" int sengine_amd_ssa_attention_noalloc(int32_t T, int32_t B, int32_t N
     return rc;
   // the K^T V kernel writes every entry the attend kernel reads: nothing to clear
   if ((rc = kv_launch(K, stream))) return rc;
+  return attend_launch(A, stream);
+}
+
+extern "C" int sengine_amd_ssa_attention_needs_kv(int32_t T, int32_t B, int32_t N, int32_t C, int32_t heads,
+                                                  int32_t workspace) {
+  return ssa_check(T, B, N, C, heads) || !fused_takes(T, B, N, heads, workspace != 0);
+}
+
+extern "C" int sengine_amd_ssa_attention(int32_t T, int32_t B, int32_t N, int32_t C, int32_t heads, float scale,
+                                         int32_t neuron, int32_t hard_reset, float tau, float v_threshold,
+                                         float v_reset, const uint32_t* q_bits, const uint32_t* k_bits,
+                                         const uint32_t* v_bits, int32_t* kv, uint32_t* out_bits,
+                                         hipStream_t stream) {
+  if (const char* why = ssa_check(T, B, N, C, heads)) return set_error(-2, why);
+  const bool fused = fused_takes(T, B, N, heads, kv != nullptr);
+  // both routes check every argument before anything is launched
+  KvLaunch K;
+  AttendLaunch A;
+  static int32_t none;  // stands for a workspace that is not needed in the checks; never dereferenced
+  int32_t* const ws = kv || !fused ? kv : &none;
+  if (const int rc = kv_setup(T, B, N, C, heads, k_bits, v_bits, ws, K)) return rc;
+  if (const int rc = attend_setup(T, B, N, C, heads, scale, neuron, hard_reset, tau, v_threshold, v_reset, q_bits, ws,
+                                  out_bits, A))
+    return rc;
+  if (fused) {
+    SsaParams p = A.p;
+    p.k = k_bits;
+    p.v = v_bits;
+    p.kv = kv;
+    return fused_launch(p, epilogue_mode(p.np, false) == EPI_LIF_HARD, stream);
+  }
+  if (const int rc = kv_launch(K, stream)) return rc;
   return attend_launch(A, stream);
 }

@@ -609,6 +609,12 @@ def real_conv_bn(s: ConvSpec, x: torch.Tensor, weight: torch.Tensor, bn_scale: t
     return out
 
 
+def attention_needs_kv(T: int, B: int, N: int, C: int, heads: int, workspace: bool = False) -> bool:
+    """Whether spiking_self_attention runs as two kernels with K^T V in a workspace between them
+    (else one kernel keeps it in LDS): of a call without `kv`, or with one (workspace=True)."""
+    return bool(_lib.load().sengine_amd_ssa_attention_needs_kv(T, B, N, C, heads, int(workspace)))
+
+
 def spiking_self_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, T: int, B: int, N: int, C: int,
                            heads: int, scale: float = 0.125, neuron: str = "lif", tau: float = 2.0,
                            v_threshold: float = 0.5, v_reset: Optional[float] = 0.0,
@@ -621,20 +627,19 @@ def spiking_self_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, T:
     for t, name in ((q, "q"), (k, "k"), (v, "v")):
         _check_req(t, n_bits, torch.int32, name)
     d = C // heads if heads else 0
-    if kv is None:
-        kv = torch.empty((T * B, heads, d, d), dtype=torch.int32, device=q.device)
-    else:
+    if kv is not None:
         _check_req(kv, T * B * heads * d * d, torch.int32, "kv")
+    elif attention_needs_kv(T, B, N, C, heads):
+        kv = torch.empty((T * B, heads, d, d), dtype=torch.int32, device=q.device)
     if out is None:
         out = torch.empty((T * B, N, C // 32), dtype=torch.int32, device=q.device)
     else:
         _check_req(out, n_bits, torch.int32, "out")
-    st = _stream(q.device)
-    check(lib.sengine_amd_ssa_kv(T, B, N, C, heads, _ptr(k), _ptr(v), _ptr(kv), st), "ssa_kv")
     hard = v_reset is not None
-    check(lib.sengine_amd_ssa_attend_neuron(T, B, N, C, heads, float(scale), neuron_code(neuron), int(hard),
-                                            float(tau), float(v_threshold), float(v_reset if hard else 0.0),
-                                            _ptr(q), _ptr(kv), _ptr(out), st), "ssa_attend_neuron")
+    check(lib.sengine_amd_ssa_attention(T, B, N, C, heads, float(scale), neuron_code(neuron), int(hard), float(tau),
+                                        float(v_threshold), float(v_reset if hard else 0.0), q.data_ptr(),
+                                        k.data_ptr(), v.data_ptr(), _ptr(kv), out.data_ptr(), _stream(q.device)),
+          "ssa_attention")
     return out
 
 

@@ -32,7 +32,7 @@ this path needs):
     launch over the concatenated weights, its spike bits split into one plane per conv -- the
     planes of one buffer, each conv's spike tensor a view of its plane;
   * FusedSpikformerAttn: the SSA core on spike bits (K^T V, then Q (K^T V) and the attention
-    LIF: two kernels), its K^T V workspace allocated in build();
+    LIF: one kernel, or two with a K^T V workspace allocated in build());
   * CuDNNPool: spike max-pool; CuBLASGemm: the head (pool + mean over T + Linear absorbed);
   * ZeroCost: views.  An unabsorbed Add / Tile / TemporalMean / GlobalAvgPool raises.
 Spike tensors live as bits, real-valued tensors as fp32 NHWC, integer activations (residual
@@ -390,7 +390,8 @@ class CUDAGraphEngine:
                     torch.from_numpy(np.ascontiguousarray(ir.weights[node.weight_info.name])).float().to(self.dev),
                     torch.from_numpy(np.ascontiguousarray(ir.weights[node.bias_info.name])).float().to(self.dev))
         # workspaces, shared by the launches that need one (they run one after another on one stream)
-        n_kv = max([self.kernels[l.nid].kv_numel for l in launches if l.kind == "attn"], default=0)
+        n_kv = max([self.kernels[l.nid].kv_numel for l in launches
+                    if l.kind == "attn" and self.kernels[l.nid].needs_kv], default=0)
         self.attn_ws = torch.empty(n_kv, dtype=torch.int32, device=self.dev) if n_kv else None
         n_hw = max([self.kernels[l.nid].workspace_numel for l in launches if l.kind == "head"], default=0)
         self.head_ws = torch.empty(n_hw, dtype=torch.int32, device=self.dev) if n_hw else None
@@ -400,9 +401,9 @@ class CUDAGraphEngine:
     @property
     def n_launches(self) -> int:
         """Kernel launches per forward (pack / unpack of a spike-input graph included; an
-        attention core is two, and so is a head whose sums are split over a workspace)."""
+        attention core with a workspace is two, and so is a head whose sums are split over one)."""
         n = sum(1 for l in self.launches if not l.skip)
-        n += sum(1 for l in self.launches if l.kind == "attn")
+        n += sum(1 for l in self.launches if l.kind == "attn" and self.kernels[l.nid].needs_kv)
         n += sum(1 for l in self.launches if l.kind == "head" and self.kernels[l.nid].workspace_numel)
         if not self.image_input:
             n += 1
@@ -423,8 +424,10 @@ class CUDAGraphEngine:
                 name = " + ".join(self.ir.nodes[i].name for i in self.ir.nodes[l.nid].extra_attrs["merged_nids"])
             if l.pair_with is not None:
                 name += " + " + self.ir.nodes[l.pair_with].name
-            if l.kind == "attn":
+            if l.kind == "attn" and self.kernels[l.nid].needs_kv:
                 names += [f"{name} (attn: key-value sums)", f"{name} (attn: attend)"]
+            elif l.kind == "attn":
+                names.append(f"{name} (attn: attend)")
             elif l.kind == "head" and self.kernels[l.nid].workspace_numel:
                 names += [f"{name} (head: partial sums)", f"{name} (head: classifier)"]
             else:
@@ -529,7 +532,7 @@ class CUDAGraphEngine:
         elif l.kind == "attn":
             kern = self.kernels[l.nid]
             q, k, v = (self._bits(t) for t in l.inputs)
-            kern(q, k, v, kv=self.attn_ws[:kern.kv_numel], out=self._bits(l.output))
+            kern(q, k, v, kv=self.attn_ws[:kern.kv_numel] if kern.needs_kv else None, out=self._bits(l.output))
         elif l.kind == "real_conv":
             sc, bi = self.bn[l.nid]
             x = self._root_fn(l.inputs[0])

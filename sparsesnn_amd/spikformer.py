@@ -194,6 +194,7 @@ class SpikformerEngine:
                          fc2=self._linear(p, pre + ".mlp.fc2", hidden, embed, 1, out_f16=f16),
                          bufs={})
             d = embed // heads
+            self.attn_kv = ops.attention_needs_kv(self.T, self.B, self.N, embed, heads, workspace=True)
             # q, k and v read the same stream: one launch over their concatenated weights, its
             # spike bits split into one plane per Linear (the fourth plane holds the padding)
             nplanes = -(-blk.qkv.spec.C_out // embed)
@@ -201,7 +202,8 @@ class SpikformerEngine:
             for j, n in enumerate(("q", "k", "v")):
                 blk.bufs[n] = blk.bufs["qkv"][j]
             blk.bufs["a"] = torch.empty(TB, self.N, embed // 32, **i32)
-            blk.bufs["kv"] = torch.empty(TB, heads, d, d, **i32)
+            if self.attn_kv:
+                blk.bufs["kv"] = torch.empty(TB, heads, d, d, **i32)
             blk.bufs["x1"] = stream_buf(P1)
             blk.bufs["h"] = torch.empty(TB, self.N, hidden // 32, **i32)
             blk.bufs["x2"] = stream_buf(P2)
@@ -322,7 +324,7 @@ class SpikformerEngine:
         ops.fused_sparse_conv_bn_lif_split(qkv.spec, x.view(-1), qkv.values, qkv.meta, qkv.scale, qkv.bias,
                                            self.embed, out=b["qkv"])
         ops.spiking_self_attention(b["q"], b["k"], b["v"], self.T, self.B, self.N, self.embed, self.heads,
-                                   v_threshold=ATTN_VTH, kv=b["kv"], out=b["a"])
+                                   v_threshold=ATTN_VTH, kv=b.get("kv"), out=b["a"])
         self._fused_add(blk.proj, b["a"], x, blk.planes_in, b["x1"], blk.planes_mid)
         self._fused(blk.fc1, b["x1"], b["h"])
         self._fused_add(blk.fc2, b["h"], b["x1"], blk.planes_mid, b["x2"], blk.planes_out)
@@ -340,9 +342,9 @@ class SpikformerEngine:
 
     @property
     def launches(self) -> int:
-        # SPS 7, 6 per block (q/k/v, SSA 2, proj, fc1, fc2), the head 1 (bit planes) or 2 (fp16
-        # stream: split sums, then the head)
-        return 7 + 6 * len(self.blocks) + (2 if self.block_input(len(self.blocks))[1] == 0 else 1)
+        # SPS 7, 5 or 6 per block (q/k/v, SSA 1 or 2, proj, fc1, fc2), the head 1 (bit planes) or 2
+        # (fp16 stream: split sums, then the head)
+        return 7 + (6 if self.blocks and self.attn_kv else 5) * len(self.blocks) + (2 if self.block_input(len(self.blocks))[1] == 0 else 1)
 
     def capture(self):
         """Capture the whole forward into a hipGraph (replayed by forward())."""
