@@ -7,6 +7,7 @@
 // MODE selects a compile-time specialisation (the epilogue's VALU work is a visible
 // share of the kernel when K_red is small):
 //   EPI_GENERIC  any neuron / reset / tau, optional per-step traces
+//   EPI_PLAIN    any neuron / reset / tau, no traces and no real-valued output (fewer registers)
 //   EPI_LIF_HARD LIF with 1/tau and 1 - 1/tau powers of two (tau = 2), hard reset, no traces
 //   EPI_IF_HARD  IF, hard reset, no traces
 // All modes compute the same values (models/neurons.py:121-146,169-184); the fast modes
@@ -16,7 +17,7 @@
 
 namespace sengine {
 
-enum { EPI_GENERIC = 0, EPI_LIF_HARD = 1, EPI_IF_HARD = 2, EPI_SHORTCUT = 3 };
+enum { EPI_GENERIC = 0, EPI_LIF_HARD = 1, EPI_IF_HARD = 2, EPI_SHORTCUT = 3, EPI_PLAIN = 4 };
 
 // One hard-reset fire step: spike = h >= v_th (VCC), v = spike ? v_reset : h, and the spike
 // shifted into `word` as its new lowest bit (word = 2*word + spike, with VCC as carry-in).
@@ -471,7 +472,8 @@ __device__ __forceinline__ void lif_epilogue(const float4_t (&acc)[T][4], bool v
   if (pre) res = *pre;
   else load_sew_res<T>(sa, M, m, F, cob, valid, res);
   float fsc[16], fbi[16], v[16];
-  const bool fold = MODE == EPI_LIF_HARD || (MODE == EPI_GENERIC && np.neuron == SENGINE_NEURON_LIF && np.pow2);
+  constexpr bool ANY = MODE == EPI_GENERIC || MODE == EPI_PLAIN;
+  const bool fold = MODE == EPI_LIF_HARD || (ANY && np.neuron == SENGINE_NEURON_LIF && np.pow2);
   float* st = state ? state + (size_t)m * F + cob : nullptr;
   const bool has_state = st != nullptr;
 #pragma unroll
@@ -584,7 +586,7 @@ __device__ __forceinline__ void lif_epilogue(const float4_t (&acc)[T][4], bool v
       }
     } else {
       float rr[16];
-      const bool real = sa.real_out != nullptr && valid;
+      const bool real = MODE == EPI_GENERIC && sa.real_out != nullptr && valid;
       if (real) {
 #pragma unroll
         for (int j = 0; j < 16; j += 4) {
@@ -609,8 +611,8 @@ __device__ __forceinline__ void lif_epilogue(const float4_t (&acc)[T][4], bool v
         const float h = neuron_charge(np, v[j], xin);
         const bool spike = h >= np.vth;
         v[j] = neuron_reset(np, h, spike);
-        if (h_trace && valid) h_trace[row + j] = h;
-        if (x_trace && valid) x_trace[row + j] = fold ? __builtin_fmaf(accv, cf.sc[j], cf.bi[j]) : xin;
+        if (MODE == EPI_GENERIC && h_trace && valid) h_trace[row + j] = h;
+        if (MODE == EPI_GENERIC && x_trace && valid) x_trace[row + j] = fold ? __builtin_fmaf(accv, cf.sc[j], cf.bi[j]) : xin;
         word |= (uint32_t)spike << j;
       }
       if (real) {

@@ -828,7 +828,7 @@ extern "C" int sengine_amd_fused_plan(const sengine_conv_lif_desc* d, int32_t fl
     else if ((choice == 0 || choice == 3) && tile3s_eligible(d))
       n = describe_tile3s(d, plan.geo, mode, buf, len);
     else
-      n = describe_lds(d, plan.geo, mode, buf, len);
+      n = describe_lds(d, plan.geo, mode, traces || shortcut, buf, len);
   } else if (plan.route == kRouteSmall) {
     n = snprintf(buf, len, "smallm<T=%d,planes=%d,out=%s,epi=%s,flat=%d>", d->T, d->weight_planes,
                  d->out_enc == SENGINE_ENC_BITS ? "bits" : "f16", kEpi[plan.mode], flat_layout(d, plan.geo) ? 1 : 0);

@@ -73,8 +73,16 @@ __device__ __forceinline__ int xcd_tile(int id, int n) {
 
 // T timesteps, PT*64 positions per workgroup, GPW 64-channel output groups per wave,
 // PL weight planes, output encoding, epilogue mode, CPS reduction chunks per LDS stage.
+//
+// Latency bound (a chunk takes about 2,400 cycles of which 512 are matrix instructions at T = 8), so
+// a second wave per SIMD counts most.  The generic epilogue's traces and real-valued rows took it
+// away from every call of that mode (T = 8: 319 registers; T = 4, GPW = 2: spilled): calls without
+// them run the plain mode, which like the hard ones is held to two waves.  Same arithmetic, same bits:
+// IF soft reset, 128->256 28x28 k5, T = 4, 16 images 448 -> 60 us; 192->320 45x37 k5 s2, T = 8,
+// 14 images 147 -> 98 us; two weight planes, LIF, 128->128 28x28 k3, 32 images 51.5 -> 33.2 us.
 template <int T, int PT, int GPW, int PL, int OUT_ENC, int MODE, int CPS>
-__global__ __launch_bounds__(256) void fused_sparse_lds_kernel(LdsParams p) {
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(MODE == EPI_GENERIC ? 1 : 2))) void fused_sparse_lds_kernel(LdsParams p) {
   constexpr int NPOS = 64 * PT;                  // positions per workgroup
   constexpr int TSTEP = 256 / NPOS;              // timesteps covered by one pass of 256 threads
   constexpr int NW = (T + TSTEP - 1) / TSTEP;    // spike words staged per thread per chunk
@@ -93,7 +101,7 @@ __global__ __launch_bounds__(256) void fused_sparse_lds_kernel(LdsParams p) {
   const int m0 = xcd_tile(blockIdx.x, gridDim.x) * NPOS;
 
   // Folded BN coefficients of this workgroup's channels (written before the first barrier).
-  const bool fold = MODE == EPI_LIF_HARD || (MODE == EPI_GENERIC && p.np.neuron == SENGINE_NEURON_LIF && p.np.pow2);
+  const bool fold = MODE == EPI_LIF_HARD || (MODE != EPI_IF_HARD && p.np.neuron == SENGINE_NEURON_LIF && p.np.pow2);
   if (tid < NCH) {
     const float sc = p.scale[G0 * 64 + tid] * p.enc_scale;  // exact: enc_scale is a power of two
     const float bi = p.bias[G0 * 64 + tid];
@@ -288,29 +296,39 @@ template <int T, int PT, int GPW, int PL, int OE, int MODE>
 static hipError_t launch_lds_t(const LdsParams& p, hipStream_t s) {
   dim3 grid((unsigned)((p.M + 64 * PT - 1) / (64 * PT)), (unsigned)(p.F / (64 * GPW)));
   if (PL == 1 && choose_cps(PL) == 2)
-    hipLaunchKernelGGL((fused_sparse_lds_kernel<T, PT, GPW, PL, OE, MODE, 2>), grid, dim3(256), 0, s, p);
+    hipLaunchKernelGGL((fused_sparse_lds_kernel<T, PT, GPW, PL, OE, MODE, PL == 1 ? 2 : 1>), grid, dim3(256), 0, s, p);
   else
     hipLaunchKernelGGL((fused_sparse_lds_kernel<T, PT, GPW, PL, OE, MODE, 1>), grid, dim3(256), 0, s, p);
   return hipGetLastError();
 }
 
+template <int T, int PT, int GPW, int PL>
+static hipError_t launch_lds_pl(const LdsParams& p, int out_enc, int mode, hipStream_t s) {
+  constexpr int BITS = SENGINE_ENC_BITS, F16 = SENGINE_ENC_F16;
+  if (out_enc != BITS && out_enc != F16) return hipErrorInvalidValue;
+  if constexpr (GPW == 1)  // choose_gpw gives the generic mode one group
+    if (mode == EPI_GENERIC)
+      return out_enc == BITS ? launch_lds_t<T, PT, GPW, PL, BITS, EPI_GENERIC>(p, s)
+                             : launch_lds_t<T, PT, GPW, PL, F16, EPI_GENERIC>(p, s);
+  if (out_enc == F16) return launch_lds_t<T, PT, GPW, PL, F16, EPI_PLAIN>(p, s);
+  if (mode == EPI_LIF_HARD) return launch_lds_t<T, PT, GPW, PL, BITS, EPI_LIF_HARD>(p, s);
+  if (mode == EPI_IF_HARD) return launch_lds_t<T, PT, GPW, PL, BITS, EPI_IF_HARD>(p, s);
+  return launch_lds_t<T, PT, GPW, PL, BITS, EPI_PLAIN>(p, s);
+}
+
 template <int T, int PT, int GPW>
 static hipError_t launch_lds_pt(const LdsParams& p, int planes, int out_enc, int mode, hipStream_t s) {
-  if (out_enc == SENGINE_ENC_BITS && mode == EPI_LIF_HARD) {
-    if (planes == 1) return launch_lds_t<T, PT, GPW, 1, SENGINE_ENC_BITS, EPI_LIF_HARD>(p, s);
-    return launch_lds_t<T, PT, GPW, 2, SENGINE_ENC_BITS, EPI_LIF_HARD>(p, s);
-  }
-  if (out_enc == SENGINE_ENC_BITS && mode == EPI_IF_HARD) {
-    if (planes == 1) return launch_lds_t<T, PT, GPW, 1, SENGINE_ENC_BITS, EPI_IF_HARD>(p, s);
-    return launch_lds_t<T, PT, GPW, 2, SENGINE_ENC_BITS, EPI_IF_HARD>(p, s);
-  }
-  if (planes == 1 && out_enc == SENGINE_ENC_BITS) return launch_lds_t<T, PT, GPW, 1, SENGINE_ENC_BITS, EPI_GENERIC>(p, s);
-  if (planes == 2 && out_enc == SENGINE_ENC_BITS) return launch_lds_t<T, PT, GPW, 2, SENGINE_ENC_BITS, EPI_GENERIC>(p, s);
-  if (planes == 1 && out_enc == SENGINE_ENC_F16) return launch_lds_t<T, PT, GPW, 1, SENGINE_ENC_F16, EPI_GENERIC>(p, s);
-  if (planes == 2 && out_enc == SENGINE_ENC_F16) return launch_lds_t<T, PT, GPW, 2, SENGINE_ENC_F16, EPI_GENERIC>(p, s);
+  if (planes == 1) return launch_lds_pl<T, PT, GPW, 1>(p, out_enc, mode, s);
+  if (planes == 2) return launch_lds_pl<T, PT, GPW, 2>(p, out_enc, mode, s);
   return hipErrorInvalidValue;
 }
 
+// The epilogue instance: traces and real-valued rows need the generic mode; otherwise the hard-reset
+// modes where they exist (spike bits) and the plain one.
+static int lds_mode(int mode, int out_enc, bool extra) {
+  if (extra) return EPI_GENERIC;
+  return mode == EPI_GENERIC || out_enc != SENGINE_ENC_BITS ? EPI_PLAIN : mode;
+}
 
 // Positions per workgroup: 64 (PT=1) measured faster than 128 on every config-1 layer
 // (more waves in flight, fewer registers); 128 only for T <= 2, where the accumulators are
@@ -324,23 +342,24 @@ static int choose_pt(int T) {
 // Output-channel groups (of 64) per wave: 2 halves the spike-bit expansion work per
 // SMFMAC (each B fragment feeds 8 instead of 4), at the cost of twice the accumulators and
 // half the workgroups.  Used when C_out % 128 == 0 and the grid still holds >= 1 wave per
-// SIMD.  SENGINE_AMD_LDS_GPW=1|2 overrides (tuning).
-static int choose_gpw(int T, int pt, int64_t M, int F) {
+// SIMD, not with the generic epilogue, which spills there (two planes, shortcut, 128->128 28x28, 32
+// images: 222 us with two groups, 69 with one).  SENGINE_AMD_LDS_GPW=1|2 overrides (tuning).
+static int choose_gpw(int T, int pt, int64_t M, int F, int mode) {
   static const int forced = env_int("SENGINE_AMD_LDS_GPW", 0);
-  if (pt != 1 || T > 4 || F % 128 != 0) return 1;
+  if (pt != 1 || T > 4 || F % 128 != 0 || mode == EPI_GENERIC) return 1;
   if (forced == 1 || forced == 2) return forced;
   const int64_t waves = ((M + 63) / 64) * (F / 128) * 4;
   return waves >= 1024 ? 2 : 1;
 }
 
-int describe_lds(const sengine_conv_lif_desc* d, const Geometry& geo, int mode, char* buf, size_t len) {
-  static const char* const kEpi[] = {"generic", "lif_hard", "if_hard"};
+int describe_lds(const sengine_conv_lif_desc* d, const Geometry& geo, int epi, bool extra, char* buf, size_t len) {
+  static const char* const kEpi[] = {"generic", "lif_hard", "if_hard", "", "plain"};
+  const int mode = lds_mode(epi, d->out_enc, extra);
   const int pt = choose_pt(d->T);
-  const int gpw = choose_gpw(d->T, pt, geo.M, d->C_out);
-  const bool fast = d->out_enc == SENGINE_ENC_BITS && (mode == EPI_LIF_HARD || mode == EPI_IF_HARD);
+  const int gpw = choose_gpw(d->T, pt, geo.M, d->C_out, mode);
   return snprintf(buf, len, "lds<T=%d,PT=%d,GPW=%d,planes=%d,out=%s,epi=%s>", d->T, d->T == 8 ? 1 : pt,
                   d->T == 8 ? 1 : gpw, d->weight_planes, d->out_enc == SENGINE_ENC_BITS ? "bits" : "f16",
-                  fast ? kEpi[mode] : "generic");
+                  kEpi[mode]);
 }
 
 hipError_t launch_fused_bits_lds(const sengine_conv_lif_desc* d, const Geometry& geo, const FusedArgs& a,
@@ -365,8 +384,9 @@ hipError_t launch_fused_bits_lds(const sengine_conv_lif_desc* d, const Geometry&
   p.enc_scale = 1.0f / kBitSpikeValue;
   p.sew = a.sew;
   const int pt = choose_pt(d->T);
-  const int gpw = choose_gpw(d->T, pt, geo.M, d->C_out);
-  const int mode = epilogue_mode(p.np, a.h_trace != nullptr || a.x_trace != nullptr || a.sew.real_out != nullptr);
+  const bool extra = a.h_trace != nullptr || a.x_trace != nullptr || a.sew.real_out != nullptr;
+  const int mode = lds_mode(epilogue_mode(p.np, extra), d->out_enc, extra);
+  const int gpw = choose_gpw(d->T, pt, geo.M, d->C_out, mode);
   const int pl = d->weight_planes, oe = d->out_enc;
 #define SENGINE_LDS_T(TT)                                                                      \
   case TT:                                                                                     \

@@ -116,7 +116,7 @@ int describe_tile3s(const sengine_conv_lif_desc* d, const Geometry& geo, int mod
 // carries which optional buffers (state, traces, residuals) the launch passes.
 int describe_tile(const sengine_conv_lif_desc* d, const Geometry& geo, int mode, bool shortcut_only,
                   const FusedArgs& a, char* buf, size_t len);
-int describe_lds(const sengine_conv_lif_desc* d, const Geometry& geo, int mode, char* buf, size_t len);
+int describe_lds(const sengine_conv_lif_desc* d, const Geometry& geo, int epi, bool extra, char* buf, size_t len);
 
 // Kernel selection for the fused op with spike-bit input: 0 = automatic (the split-K
 // small-M kernel for small outputs, else the tile kernel where eligible, else the
