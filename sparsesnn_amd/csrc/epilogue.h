@@ -19,24 +19,50 @@ namespace sengine {
 
 enum { EPI_GENERIC = 0, EPI_LIF_HARD = 1, EPI_IF_HARD = 2, EPI_SHORTCUT = 3, EPI_PLAIN = 4 };
 
-// One hard-reset fire step: spike = h >= v_th (VCC), v = spike ? v_reset : h, and the spike
-// shifted into `word` as its new lowest bit (word = 2*word + spike, with VCC as carry-in).
-// Three VALU ops; the compiler's form needs a separate select to materialise the bit.
-__device__ __forceinline__ void fire_hard(float h, float vth, float vreset, float& v, uint32_t& word) {
-  asm("v_cmp_le_f32_e32 vcc, %[th], %[h]\n\t"
-      "v_cndmask_b32_e32 %[v], %[h], %[vr], vcc\n\t"
-      "v_addc_co_u32_e32 %[w], vcc, %[w], %[w], vcc"
-      : [v] "=&v"(v), [w] "+v"(word)
-      : [h] "v"(h), [th] "s"(vth), [vr] "v"(vreset)
+// Hard-reset fire steps of four neurons.  Each h holds a charge and becomes the membrane: spike =
+// h >= v_th, h = spike ? v_reset : h, and the spike is shifted into `word` as its new lowest bit
+// (word = 2*word + spike, the compare as carry-in), h0's first.  Three VALU ops a neuron; the
+// compiler's form needs a separate select to materialise the bit.
+//
+// gfx950 wants two wait states between a VALU write of VCC or an SGPR and a VALU read of it, and the
+// compiler puts none inside an asm block: every compare has its own SGPR pair and three other
+// instructions between it and its first reader.  (One neuron at a time through VCC, as these blocks
+// were, has none or one.)  Filling the waits with neighbours costs no issue slots, where the
+// compiler's s_nop after each compare would.
+__device__ __forceinline__ void fire_hard4(float& h0, float& h1, float& h2, float& h3, float vth, float vreset,
+                                           uint32_t& word) {
+  uint64_t s1, s2, s3;
+  asm("v_cmp_le_f32_e32 vcc, %[th], %[h0]\n\t"
+      "v_cmp_le_f32_e64 %[s1], %[th], %[h1]\n\t"
+      "v_cmp_le_f32_e64 %[s2], %[th], %[h2]\n\t"
+      "v_cmp_le_f32_e64 %[s3], %[th], %[h3]\n\t"
+      "v_cndmask_b32_e32 %[h0], %[h0], %[vr], vcc\n\t"
+      "v_cndmask_b32_e64 %[h1], %[h1], %[vr], %[s1]\n\t"
+      "v_cndmask_b32_e64 %[h2], %[h2], %[vr], %[s2]\n\t"
+      "v_cndmask_b32_e64 %[h3], %[h3], %[vr], %[s3]\n\t"
+      "v_addc_co_u32_e32 %[w], vcc, %[w], %[w], vcc\n\t"
+      "v_addc_co_u32_e64 %[w], vcc, %[w], %[w], %[s1]\n\t"
+      "v_addc_co_u32_e64 %[w], vcc, %[w], %[w], %[s2]\n\t"
+      "v_addc_co_u32_e64 %[w], vcc, %[w], %[w], %[s3]"
+      : [h0] "+v"(h0), [h1] "+v"(h1), [h2] "+v"(h2), [h3] "+v"(h3), [w] "+v"(word), [s1] "=&s"(s1), [s2] "=&s"(s2),
+        [s3] "=&s"(s3)
+      : [th] "s"(vth), [vr] "v"(vreset)
       : "vcc");
 }
 
-// Same without the reset (last timestep, membrane not kept).
-__device__ __forceinline__ void fire_only(float h, float vth, uint32_t& word) {
-  asm("v_cmp_le_f32_e32 vcc, %[th], %[h]\n\t"
-      "v_addc_co_u32_e32 %[w], vcc, %[w], %[w], vcc"
-      : [w] "+v"(word)
-      : [h] "v"(h), [th] "s"(vth)
+// The spike bits alone (last timestep, membrane not kept).
+__device__ __forceinline__ void fire_only4(float h0, float h1, float h2, float h3, float vth, uint32_t& word) {
+  uint64_t s1, s2, s3;
+  asm("v_cmp_le_f32_e32 vcc, %[th], %[h0]\n\t"
+      "v_cmp_le_f32_e64 %[s1], %[th], %[h1]\n\t"
+      "v_cmp_le_f32_e64 %[s2], %[th], %[h2]\n\t"
+      "v_cmp_le_f32_e64 %[s3], %[th], %[h3]\n\t"
+      "v_addc_co_u32_e32 %[w], vcc, %[w], %[w], vcc\n\t"
+      "v_addc_co_u32_e64 %[w], vcc, %[w], %[w], %[s1]\n\t"
+      "v_addc_co_u32_e64 %[w], vcc, %[w], %[w], %[s2]\n\t"
+      "v_addc_co_u32_e64 %[w], vcc, %[w], %[w], %[s3]"
+      : [w] "+v"(word), [s1] "=&s"(s1), [s2] "=&s"(s2), [s3] "=&s"(s3)
+      : [h0] "v"(h0), [h1] "v"(h1), [h2] "v"(h2), [h3] "v"(h3), [th] "s"(vth)
       : "vcc");
 }
 
@@ -197,14 +223,16 @@ __device__ __forceinline__ void fast_epilogue_stateless(const float4_t (&acc)[T]
   for (int t = 0; t < T; ++t) {
     uint32_t word = 0;
 #pragma unroll
-    for (int j = 15; j >= 0; --j) {
-      const float xin = __builtin_fmaf(acc[t][j >> 2][j & 3], fsc[j], fbi[j]);
-      const float h = t == 0 ? xin
-                             : (MODE == EPI_LIF_HARD ? __builtin_fmaf(v[j], np.decay, xin) : __fadd_rn(v[j], xin));
+    for (int j4 = 12; j4 >= 0; j4 -= 4) {
+#pragma unroll
+      for (int j = j4; j < j4 + 4; ++j) {
+        const float xin = __builtin_fmaf(acc[t][j >> 2][j & 3], fsc[j], fbi[j]);
+        v[j] = t == 0 ? xin : (MODE == EPI_LIF_HARD ? __builtin_fmaf(v[j], np.decay, xin) : __fadd_rn(v[j], xin));
+      }
       if (t + 1 < T)
-        fire_hard(h, np.vth, vreset, v[j], word);
+        fire_hard4(v[j4 + 3], v[j4 + 2], v[j4 + 1], v[j4], np.vth, vreset, word);
       else
-        fire_only(h, np.vth, word);
+        fire_only4(v[j4 + 3], v[j4 + 2], v[j4 + 1], v[j4], np.vth, word);
     }
     if (!valid) continue;
     const size_t row = ((size_t)t * M + m) * F + cob;
@@ -260,16 +288,15 @@ __device__ __forceinline__ void lean_epilogue_stateless(const float4_t (&acc)[4]
       const float4_t s4 = *reinterpret_cast<const float4_t*>(fsc + j4);
       const float4_t b4 = *reinterpret_cast<const float4_t*>(fbi + j4);
 #pragma unroll
-      for (int e = 3; e >= 0; --e) {
+      for (int e = 0; e < 4; ++e) {
         const int j = j4 + e;
         const float xin = __builtin_fmaf(acc[t][j >> 2][j & 3], s4[e], b4[e]);
-        const float h = t == 0 ? xin
-                               : (MODE == EPI_LIF_HARD ? __builtin_fmaf(v[j], np.decay, xin) : __fadd_rn(v[j], xin));
-        if (t + 1 < T)
-          fire_hard(h, np.vth, np.vreset, v[j], word);
-        else
-          fire_only(h, np.vth, word);
+        v[j] = t == 0 ? xin : (MODE == EPI_LIF_HARD ? __builtin_fmaf(v[j], np.decay, xin) : __fadd_rn(v[j], xin));
       }
+      if (t + 1 < T)
+        fire_hard4(v[j4 + 3], v[j4 + 2], v[j4 + 1], v[j4], np.vth, np.vreset, word);
+      else
+        fire_only4(v[j4 + 3], v[j4 + 2], v[j4 + 1], v[j4], np.vth, word);
     }
     if (!valid) continue;
     if constexpr (OUT_ENC == SENGINE_ENC_BITS) {
@@ -320,12 +347,12 @@ __device__ __forceinline__ void lean_epilogue_state(const float4_t (&acc)[4][4],
       const float4_t s4 = *reinterpret_cast<const float4_t*>(fsc + j4);
       const float4_t b4 = *reinterpret_cast<const float4_t*>(fbi + j4);
 #pragma unroll
-      for (int e = 3; e >= 0; --e) {
+      for (int e = 0; e < 4; ++e) {
         const int j = j4 + e;
         const float xin = __builtin_fmaf(acc[t][j >> 2][j & 3], s4[e], b4[e]);
-        const float h = MODE == EPI_LIF_HARD ? __builtin_fmaf(v[j], np.decay, xin) : __fadd_rn(v[j], xin);
-        fire_hard(h, np.vth, np.vreset, v[j], word);
+        v[j] = MODE == EPI_LIF_HARD ? __builtin_fmaf(v[j], np.decay, xin) : __fadd_rn(v[j], xin);
       }
+      fire_hard4(v[j4 + 3], v[j4 + 2], v[j4 + 1], v[j4], np.vth, np.vreset, word);
     }
     if (!valid) continue;
     if (OUT_ENC == SENGINE_ENC_BITS) {
@@ -578,11 +605,14 @@ __device__ __forceinline__ void lif_epilogue(const float4_t (&acc)[T][4], bool v
       // reset is computed at every step (the last one is simply not stored).  Channels
       // 15..0 so that channel j ends in bit j of the shifted-in word.
 #pragma unroll
-      for (int j = 15; j >= 0; --j) {
-        const float xin = __builtin_fmaf(acc[t][j >> 2][j & 3], fsc[j], fbi[j]);
-        const float h = MODE == EPI_LIF_HARD ? __builtin_fmaf(v[j], np.decay, xin)  // v*decay exact: one rounding
-                                             : __fadd_rn(v[j], xin);
-        fire_hard(h, np.vth, vreset, v[j], word);
+      for (int j4 = 12; j4 >= 0; j4 -= 4) {
+#pragma unroll
+        for (int j = j4; j < j4 + 4; ++j) {
+          const float xin = __builtin_fmaf(acc[t][j >> 2][j & 3], fsc[j], fbi[j]);
+          v[j] = MODE == EPI_LIF_HARD ? __builtin_fmaf(v[j], np.decay, xin)  // v*decay exact: one rounding
+                                      : __fadd_rn(v[j], xin);
+        }
+        fire_hard4(v[j4 + 3], v[j4 + 2], v[j4 + 1], v[j4], np.vth, vreset, word);
       }
     } else {
       float rr[16];

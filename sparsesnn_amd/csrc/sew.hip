@@ -3,6 +3,7 @@
 // T, max-pooling of spike bits, and the pooled / time-averaged Linear head.  All of them
 // are small next to the fused convolutions; they are HBM- or launch-bound.
 #include "common.h"
+#include "epilogue.h"
 #include "internal.h"
 
 namespace sengine {
@@ -335,17 +336,6 @@ __global__ __launch_bounds__(kStemPix * 16 / CPT) void stem_conv_bn_lds_kernel(S
   }
 }
 
-// One neuron step of a hard-reset LIF / IF on charge h = fma(v, dec, x): the spike bit is shifted
-// into `word` from below (word = 2 word + spike) and v becomes vreset where it fired.
-__device__ __forceinline__ void stem_fire(float h, float vth, float vreset, float& v, uint32_t& word) {
-  asm("v_cmp_le_f32_e32 vcc, %[th], %[h]\n\t"
-      "v_cndmask_b32_e32 %[v], %[h], %[vr], vcc\n\t"
-      "v_addc_co_u32_e32 %[w], vcc, %[w], %[w], vcc"
-      : [v] "=&v"(v), [w] "+v"(word)
-      : [h] "v"(h), [th] "v"(vth), [vr] "v"(vreset)
-      : "vcc");
-}
-
 // Stem + neuron on the fp32 matrix cores (v_mfma_f32_16x16x4_f32, 4 taps per instruction):
 // the convolution as a GEMM of channels x (C_ * KH_ * KW_ taps, HWIO order: tap k =
 // (kh * KW + kw) * C + c, zero weights past the last tap) x (output pixels).  Workgroup = (image
@@ -471,18 +461,21 @@ __global__ __launch_bounds__(256) void stem_mfma_kernel(StemParams p) {
 #pragma unroll
       for (int k = 0; k < 4; ++k)  // steps past T run and are not stored
 #pragma unroll
-        for (int c = 0; c < CT; ++c)
+        for (int c = 0; c < CT; ++c) {
+          if (FASTN) {
 #pragma unroll
-          for (int r = 3; r >= 0; --r) {
-            if (FASTN) {
-              stem_fire(__builtin_fmaf(v[c][r], dec, xo[c][r]), p.np.vth, p.np.vreset, v[c][r], nib[c]);
-            } else {
+            for (int r = 0; r < 4; ++r) v[c][r] = __builtin_fmaf(v[c][r], dec, xo[c][r]);
+            fire_hard4(v[c][3], v[c][2], v[c][1], v[c][0], p.np.vth, p.np.vreset, nib[c]);
+          } else {
+#pragma unroll
+            for (int r = 3; r >= 0; --r) {
               const float h = neuron_charge(p.np, v[c][r], xo[c][r]);
               const bool spike = h >= p.np.vth;
               v[c][r] = neuron_reset(p.np, h, spike);
               nib[c] = 2 * nib[c] + (uint32_t)spike;
             }
           }
+        }
       // nib: step t0 + k in nibble 3 - k.  Lane group q ends with step t0 + 3 - q, the nibble of
       // source group g at bits 4g of the tile's 16.
       const int t = t0 + 3 - q;

@@ -573,20 +573,23 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
         }
         // neuron on x[token][j = 16 jt + 4 q + e], spikes shifted in so that e = 0 ends lowest
 #pragma unroll
-        for (int jt = 0; jt < JT; ++jt)
+        for (int jt = 0; jt < JT; ++jt) {
+          if (FASTN) {
 #pragma unroll
-          for (int e = 3; e >= 0; --e) {
-            const float xv = acc[jt][e];
-            if (FASTN) {
-              const float hh = __builtin_fmaf(v[jt][e], p.np.decay, xv);  // v*decay exact: one rounding
-              fire_hard(hh, p.np.vth, p.np.vreset, v[jt][e], nib[jt]);
-            } else {
+            for (int e = 0; e < 4; ++e)
+              v[jt][e] = __builtin_fmaf(v[jt][e], p.np.decay, acc[jt][e]);  // v*decay exact: one rounding
+            fire_hard4(v[jt][3], v[jt][2], v[jt][1], v[jt][0], p.np.vth, p.np.vreset, nib[jt]);
+          } else {
+#pragma unroll
+            for (int e = 3; e >= 0; --e) {
+              const float xv = acc[jt][e];
               const float hh = neuron_charge(p.np, v[jt][e], fold ? xv * p.np.rtau : xv);
               const bool spike = hh >= p.np.vth;
               v[jt][e] = neuron_reset(p.np, hh, spike);
               nib[jt] = 2 * nib[jt] + (uint32_t)spike;
             }
           }
+        }
       }
       // nib: step t0 + k in nibble 3 - k; lane group q ends with the words of step t0 + 3 - q
       const int t = t0 + 3 - q;
