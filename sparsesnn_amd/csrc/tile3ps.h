@@ -176,26 +176,31 @@ void fused_tile3ps_kernel(TileParams p, int ncb) {
     // f + 1's first operands into set 1.
     const bool pc = PAIR && c == nfull;
     uint2 fr[2][4];
+    // Fragments of step (i, t), one step ahead of their use.  Asm reads, waited for by hand, count as
+    // written where the block stands: sound while the code between a read and its wait is straight.
+    // The paired chunk's tests put joins there, where the compiler copied values that had not arrived,
+    // so PAIR reads with ordinary loads and the compiler's waits (96 -> 192 channels padded to 128,
+    // 224x224, 32 images: 1,239 us; 1,230-1,294 with asm reads).
     // (the LDS base is an argument: asm operands do not capture through the lambda)
-    auto issue = [](int step, uint2 (&fq)[4], uint32_t l0, bool pr) __attribute__((always_inline)) {
+    auto issue = [bbase, pc](int step, uint2 (&fq)[4], uint32_t l0) __attribute__((always_inline)) {
       const int i = step / T, t = step - (step / T) * T;
-      const int oa = (t * TS + (i / 3) * Gm::HC + (i % 3)) * 8;
-      if (PAIR && pr) {
+      const int tap = t * TS + (i / 3) * Gm::HC + (i % 3);
+      if constexpr (PAIR) {
         const int ta = 2 * i < 9 ? 2 * i : 8, tb = 2 * i + 1 < 9 ? 2 * i + 1 : 8;
-        const int pa = (t * TS + (ta / 3) * Gm::HC + (ta % 3)) * 8;
-        const int pb = (t * TS + (tb / 3) * Gm::HC + (tb % 3)) * 8;
-        asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(fq[0]) : "v"(l0), "i"(pa));
-        asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(fq[1]) : "v"(l0), "i"(pa + 4 * NPIX * 8));
-        asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(fq[2]) : "v"(l0), "i"(pb));
-        asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(fq[3]) : "v"(l0), "i"(pb + 4 * NPIX * 8));
+        const uint2* lo = &sB[bbase + (pc ? t * TS + (ta / 3) * Gm::HC + (ta % 3) : tap)];
+        const uint2* hi = &sB[bbase + (pc ? t * TS + (tb / 3) * Gm::HC + (tb % 3) : tap + 2 * NPIX)];
+        fq[0] = lo[0];
+        fq[1] = lo[4 * NPIX];
+        fq[2] = hi[0];
+        fq[3] = hi[4 * NPIX];
       } else {
-        asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(fq[0]) : "v"(l0), "i"(oa));
-        asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(fq[1]) : "v"(l0), "i"(oa + 4 * NPIX * 8));
-        asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(fq[2]) : "v"(l0), "i"(oa + 2 * NPIX * 8));
-        asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(fq[3]) : "v"(l0), "i"(oa + 6 * NPIX * 8));
+        asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(fq[0]) : "v"(l0), "i"(tap * 8));
+        asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(fq[1]) : "v"(l0), "i"((tap + 4 * NPIX) * 8));
+        asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(fq[2]) : "v"(l0), "i"((tap + 2 * NPIX) * 8));
+        asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(fq[3]) : "v"(l0), "i"((tap + 6 * NPIX) * 8));
       }
     };
-    issue(0, fr[0], lds0, pc);
+    issue(0, fr[0], lds0);
 #pragma unroll
     for (int i = 0; i < 9; ++i) {
       if (PAIR && i >= 5 && pc) continue;
@@ -208,9 +213,10 @@ void fused_tile3ps_kernel(TileParams p, int ncb) {
         const int step = i * T + t;
         uint2(&fq)[4] = fr[step & 1];
         if (!(last && t == T - 1)) {
-          issue(step + 1, fr[(step + 1) & 1], lds0, pc);
-          asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(fq[0]), "+v"(fq[1]), "+v"(fq[2]), "+v"(fq[3]) :: "memory");
-        } else {
+          issue(step + 1, fr[(step + 1) & 1], lds0);
+          if constexpr (!PAIR)
+            asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(fq[0]), "+v"(fq[1]), "+v"(fq[2]), "+v"(fq[3]) :: "memory");
+        } else if constexpr (!PAIR) {
           asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fq[0]), "+v"(fq[1]), "+v"(fq[2]), "+v"(fq[3]) :: "memory");
         }
         const half16_t bf = __builtin_bit_cast(
