@@ -18,6 +18,7 @@
 //                      from bits, one fp32 accumulator), the neuron over T in
 //                      registers, 16 output channels of a token assembled across lanes
 //                      and stored as one u16.
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -735,16 +736,24 @@ int attend_launch(AttendLaunch& L, hipStream_t stream) {
   return (int)hipLaunchKernel(L.fn, dim3((unsigned)(L.p.B * L.p.H * L.splits)), dim3(256), args, L.lds, stream);
 }
 
-// Whether the one-workgroup-per-(b, head) kernel takes a call: long token grids of few (b, head)
-// pairs stay with the two kernels, which split the tokens over the chip.  Measured (T = 4, C = 384, 8
-// heads, two kernels / fused, us): 196 tokens, 8 pairs 19.6 / 13.6, 256 pairs 39.5 / 14.6; 784 tokens
-// (C = 512), 64 pairs 44.6 / 37.6; 3,136 tokens, 8 pairs 59.6 / 85.9, 64 pairs 82.8 / 86.8, 128 pairs
-// 97.6 / 88.7, 256 pairs 135.5 / 92.4.
-// A caller that brings a workspace (an engine plans its launches with it) gets the two kernels for
-// few pairs at any token count.
-bool fused_takes(int T, int B, int N, int heads, bool workspace) {
+// Whether the one-workgroup-per-(b, head) kernel takes a call.  Its time is that of one workgroup,
+// whatever their number up to one per CU: about 4 us + 0.025 us T d + 0.13 ns N T d.  The two kernels
+// take 14 to 25 us however small the call, split long token grids over the chip, and grow with the
+// pairs.  So the line is N T d against the pairs, read off 1,766 shapes (T 1-8, head dims 16-64, 16 to
+// 3,136 tokens, 1 to 128 pairs; a 16-wide head costs what a 32-wide one does).  us, two kernels / one:
+//   T = 4, d = 48, 8 pairs: 196 tokens 19.6 / 13.6, 400 21.3 / 18.4, 576 22.6 / 22.3, 784 24.6 / 28.8,
+//   3,136 59.2 / 86.1;  32 pairs: 784 tokens 29.0 / 28.7, 1,024 29.7 / 34.6;  64 pairs: 1,024 38.7 /
+//   34.6, 3,136 82.2 / 87.3;  96 pairs: 3,136 102.7 / 89.4, 6,272 171.2 / 172.9
+//   T = 8, d = 64: 8 pairs, 64 tokens 25.3 / 17.8, 196 27.2 / 29.9, 576 30.0 / 54.6;  64 pairs, 784
+//   tokens 80.5 / 70.2;  88 pairs, 768 tokens 106 / 70
+//   T = 1, d = 32, 3,136 tokens: 4 pairs 39.3 / 18.2, one pair 17.6 / 17.9
+// Below eight pairs a caller that brings a workspace (an engine plans its launches with it) keeps the
+// two launches that its launch count states.
+bool fused_takes(int T, int B, int N, int d, int heads, bool workspace) {
   if (T != 1 && T != 2 && T != 4 && T != 8) return false;
-  return (N <= 768 && !workspace) || (int64_t)B * heads >= 96;
+  const int64_t pairs = (int64_t)B * heads, td = (int64_t)T * std::max(d, 32);
+  if (workspace && pairs < 8) return false;
+  return pairs >= 80 || N * td <= 2304 * (32 + pairs) || (td <= 96 && pairs >= 4);
 }
 
 template <int D, int T>
@@ -857,7 +866,7 @@ extern "C" int sengine_amd_ssa_attention_noalloc(int32_t T, int32_t B, int32_t N
 
 extern "C" int sengine_amd_ssa_attention_needs_kv(int32_t T, int32_t B, int32_t N, int32_t C, int32_t heads,
                                                   int32_t workspace) {
-  return ssa_check(T, B, N, C, heads) || !fused_takes(T, B, N, heads, workspace != 0);
+  return ssa_check(T, B, N, C, heads) || !fused_takes(T, B, N, C / heads, heads, workspace != 0);
 }
 
 extern "C" int sengine_amd_ssa_attention(int32_t T, int32_t B, int32_t N, int32_t C, int32_t heads, float scale,
@@ -866,7 +875,7 @@ extern "C" int sengine_amd_ssa_attention(int32_t T, int32_t B, int32_t N, int32_
                                          const uint32_t* v_bits, int32_t* kv, uint32_t* out_bits,
                                          hipStream_t stream) {
   if (const char* why = ssa_check(T, B, N, C, heads)) return set_error(-2, why);
-  const bool fused = fused_takes(T, B, N, heads, kv != nullptr);
+  const bool fused = fused_takes(T, B, N, C / heads, heads, kv != nullptr);
   // both routes check every argument before anything is launched
   KvLaunch K;
   AttendLaunch A;

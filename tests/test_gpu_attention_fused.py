@@ -58,10 +58,7 @@ def test_fused_attention_exact(dev, T, B, N, C, heads, p, neuron, tau, v_reset):
     assert torch.equal(out.cpu(), ref) and torch.equal(ws.cpu(), kv.int())
 
 
-def test_long_grids_of_few_heads_keep_two_kernels(dev):
-    assert ops.attention_needs_kv(4, 1, 3136, 384, 8) and not ops.attention_needs_kv(4, 1, 768, 384, 8)
-    assert ops.attention_needs_kv(4, 11, 196, 384, 8, workspace=True)
-    assert not ops.attention_needs_kv(4, 12, 3136, 384, 8, workspace=True)
+def test_attention_refusals_of_the_one_kernel(dev):
     with pytest.raises(ops.SEngineError):  # what the two kernels refuse, the one refuses: scale not a power of two
         t = torch.zeros(4, 16, 2, dtype=torch.int32, device=dev)
         ops.spiking_self_attention(t, t, t, 4, 1, 16, 64, 4, scale=0.3)
