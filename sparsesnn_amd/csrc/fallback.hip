@@ -263,7 +263,7 @@ __device__ __forceinline__ uint32_t or_over_8_lanes(uint32_t x) {
 // Four elements per thread (16-byte accesses; the pointers and n allow them), the inputs of up to
 // four timesteps in flight together.  Bound by HBM: one fp32 read per element and step.  The spike
 // words of four steps are stored by four different lanes of each eight-lane run in one instruction.
-// 3.2M elements x 4 steps (51 MB): 16.8 -> 10.7 us.
+// 3.2M elements x 4 steps (51 MB): 16.7 -> 11.7 us against the form above, 1.6M 6.7 -> 4.9.
 template <int OUT_ENC>
 __global__ __launch_bounds__(256) void multistep_neuron4_kernel(NeuronKernelParams p) {
   constexpr int TC = 4;
@@ -277,8 +277,10 @@ __global__ __launch_bounds__(256) void multistep_neuron4_kernel(NeuronKernelPara
   for (int t0 = 0; t0 < p.T; t0 += TC) {
     float4_t x[TC];
 #pragma unroll
-    for (int k = 0; k < TC; ++k)
-      x[k] = *reinterpret_cast<const float4_t*>(p.x + (int64_t)min(t0 + k, p.T - 1) * p.n + sc);
+    for (int k = 0; k < TC; ++k) {
+      if (t0 + k >= p.T) break;
+      x[k] = *reinterpret_cast<const float4_t*>(p.x + (int64_t)(t0 + k) * p.n + sc);
+    }
     uint32_t mine = 0;
 #pragma unroll
     for (int k = 0; k < TC; ++k) {
@@ -420,8 +422,12 @@ extern "C" int sengine_amd_multistep_neuron(int32_t T, int64_t n, int32_t neuron
     return set_error(-2, "multistep_neuron: out_enc must be BITS or F16");
   NeuronKernelParams p{x, state, static_cast<uint8_t*>(spikes), h_trace, n, T,
                        make_neuron_params(neuron, hard_reset, tau, v_threshold, v_reset)};
-  // 16-byte rows: every timestep's row and every buffer on a 16-byte boundary (fp16 spikes: 8)
-  if (n % 4 == 0 && aligned16(x) && aligned16(state) && aligned16(h_trace) &&
+  // Four elements per thread once one each is more threads than the chip holds (2,048 per CU) and
+  // would take a second round; below, four neurons in one thread are only a longer chain.  T = 4, bits,
+  // one element / four, us: 32,768 elements 2.6 / 3.4, 393,216 3.1 / 3.7, 524,288 3.4 / 3.8, 655,360
+  // 4.2 / 4.0, 1,605,632 6.7 / 4.9.  Needs 16-byte rows: every timestep's row and every buffer on a
+  // 16-byte boundary (fp16 spikes: 8).
+  if (n > 2048ll * device_cus() && n % 4 == 0 && aligned16(x) && aligned16(state) && aligned16(h_trace) &&
       (out_enc == SENGINE_ENC_BITS || reinterpret_cast<uintptr_t>(spikes) % 8 == 0)) {
     const dim3 grid4((unsigned)((n / 4 + 255) / 256));
     if (out_enc == SENGINE_ENC_BITS)

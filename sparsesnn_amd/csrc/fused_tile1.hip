@@ -8,6 +8,8 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <atomic>
+
 namespace sengine {
 
 hipError_t launch_tile1(const TileParams& p, int T, int gpw, int oe, int mode, hipStream_t s) {
@@ -155,18 +157,16 @@ static int tile_epilogue_mode(const sengine_conv_lif_desc* d, const TileChoice& 
   return mode;
 }
 
-// Compute units of the current device (cached per device; the persistent 1x1 kernel sizes its
-// grid to the resident workgroups).
-static int device_cus() {
-  static int cus[64] = {};
+int device_cus() {
+  static std::atomic<int> cus[64] = {};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cus[dev] <= 0) {
-    int n = 0;
+  int n = cus[dev];
+  if (n <= 0) {
     if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
     cus[dev] = n;
   }
-  return cus[dev];
+  return n;
 }
 
 // The persistent 1x1 kernel (tile1ps.h) serves the token Linears when a layer is what it is

@@ -118,6 +118,9 @@ int describe_tile(const sengine_conv_lif_desc* d, const Geometry& geo, int mode,
                   const FusedArgs& a, char* buf, size_t len);
 int describe_lds(const sengine_conv_lif_desc* d, const Geometry& geo, int epi, bool extra, char* buf, size_t len);
 
+// Compute units of the current device (looked up once per device; 256 where there is none).
+int device_cus();
+
 // Kernel selection for the fused op with spike-bit input: 0 = automatic (the split-K
 // small-M kernel for small outputs, else the tile kernel where eligible, else the
 // LDS-staged kernel), 1 = always the direct-gather kernel, 2 = the LDS-staged kernel,

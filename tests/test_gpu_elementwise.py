@@ -23,7 +23,12 @@ def _shifted(t, off):
 @pytest.mark.parametrize("T,n,off,enc", [(1, 32, 0, ops.ENC_BITS), (3, 1056, 0, ops.ENC_BITS),
                                          (4, 64 * 37, 0, ops.ENC_BITS), (4, 64 * 37, 1, ops.ENC_BITS),
                                          (9, 4096, 0, ops.ENC_BITS), (4, 1028, 0, ops.ENC_F16),
-                                         (5, 1030, 0, ops.ENC_F16), (4, 1028, 2, ops.ENC_F16)])
+                                         (5, 1030, 0, ops.ENC_F16), (4, 1028, 2, ops.ENC_F16),
+                                         # four elements per thread: more than the chip's 524,288 threads
+                                         (4, 524288, 0, ops.ENC_BITS), (1, 524320, 0, ops.ENC_BITS),
+                                         (6, 524320, 0, ops.ENC_BITS), (4, 524320, 1, ops.ENC_BITS),
+                                         (3, 524292, 0, ops.ENC_F16), (5, 524294, 0, ops.ENC_F16),
+                                         (4, 524292, 2, ops.ENC_F16)])
 def test_neuron_forms(dev, neuron, tau, v_reset, T, n, off, enc):
     g = torch.Generator().manual_seed(T * n + off)
     x = torch.randn((T, n), generator=g) * 1.5 + 0.5
