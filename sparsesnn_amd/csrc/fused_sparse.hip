@@ -313,7 +313,7 @@ __device__ __forceinline__ void smallm_body(const FusedParams& p, const int bx, 
 // runs BN and the neuron over T for them from those registers (membrane state included), and the
 // spike bits meet in LDS: thread (t, lane) then holds the 4 NA channels of a position and step,
 // adds the SEW residual and stores.  NA = 2 (a workgroup of 32 channels, byte stores) doubles the
-// workgroups where 64-channel ones leave CUs idle.  Operands are requested D - 1 chunks ahead in a
+// workgroups where that adds no round over the chip (small_split).  Operands are requested D - 1 chunks ahead in a
 // ring that is unrolled, not moved.  Same sums in the same order.
 //
 // Latency bound (a few chunks per wave): what counts is the chain launch -> operands -> sum ->
@@ -542,18 +542,26 @@ __global__ __launch_bounds__(64 * kSmallWaves) void fused_smallms_pair_kernel(Fu
   smallms_body<T, PLANES, MODE, NA>(p, (int)blockIdx.x, second ? (int)blockIdx.y - g0 : (int)blockIdx.y);
 }
 
-// 64-channel workgroups of the spread form below this many (one per CU) become pairs of 32-channel
-// ones: 64 workgroups (64->64 32x32, one image, two weight planes) 5.4 -> 4.5 us, 104 (512->512
-// 7x7, four images) 12.3 -> 11.0; but 256 (64->64 8x8, 64 images) 5.3 -> 7.2, since a pair expands
-// the same spikes twice.
-constexpr int64_t kSmallSplitBelow = 256;
+// Whether `wgs` 64-channel workgroups of the spread form run as twice as many 32-channel ones.  Each CU
+// holds one of the former; a pair expands the same spikes twice, so a 32-channel workgroup takes 0.8 to
+// 0.9 of the time (two thirds at T * planes = 16, where the 64-channel one spills 120 bytes a lane) and
+// pays where the rounds over the chip stay what they are: as long as every one has a CU of its own, and
+// at T * planes = 16 also as three rounds against two.  Measured, 32- / 64-channel workgroups, us:
+// 64->64 16x16 k3, T = 4: 128 4.5 / 5.1, 160 6.9 / 5.2, 256 7.0 / 5.2;  512->512 4x4 k3: 128 10.5 / 11.7,
+// 136 18.6 / 11.7;  128->128 9x9 k5, T = 8, two planes: 112 13.4 / 20.6, 132 24.2 / 20.8, 284 34.8 / 37.1;
+// 128->256 k1, T = 8, two planes: 392 15.3 / 12.5.
+static bool small_split(int64_t wgs, int T, int planes) {
+  const int64_t cus = device_cus();
+  const int64_t split = (2 * wgs + cus - 1) / cus, whole = (wgs + cus - 1) / cus;
+  return split <= whole || (T * planes == 16 && 2 * split <= 3 * whole);
+}
 
 template <int T>
 static hipError_t launch_smallm(const FusedParams& p, int out_enc, int planes, int mode, hipStream_t s) {
   const dim3 grid((unsigned)((p.M + 15) / 16), (unsigned)(p.F / 64));
   const dim3 block(64 * kSmallWaves);
   if (mode != EPI_GENERIC) {  // spike-bit output (plan_fused)
-    const bool split = (int64_t)grid.x * grid.y < kSmallSplitBelow;
+    const bool split = small_split((int64_t)grid.x * grid.y, T, planes);
     const dim3 grid2(grid.x, grid.y * 2);
 #define SENGINE_SMALLMS_CASE(PL, MD)                                                             \
   if (planes == PL && mode == MD) {                                                              \
@@ -590,7 +598,7 @@ static hipError_t launch_smallm_pair(const FusedParams& p0, const FusedParams& p
   const dim3 grid((unsigned)((std::max(p0.M, p1.M) + 15) / 16), (unsigned)(g0 + p1.F / 64));
   const dim3 block(64 * kSmallWaves);
   if (mode != EPI_GENERIC) {
-    const bool split = (int64_t)grid.x * grid.y < kSmallSplitBelow;
+    const bool split = small_split((int64_t)grid.x * grid.y, T, planes);
     const dim3 grid2(grid.x, grid.y * 2);
 #define SENGINE_SMALLMS_PAIR_CASE(PL, MD)                                                                   \
   if (planes == PL && mode == MD) {                                                                         \
@@ -830,8 +838,10 @@ extern "C" int sengine_amd_fused_plan(const sengine_conv_lif_desc* d, int32_t fl
     else
       n = describe_lds(d, plan.geo, mode, traces || shortcut, buf, len);
   } else if (plan.route == kRouteSmall) {
-    n = snprintf(buf, len, "smallm<T=%d,planes=%d,out=%s,epi=%s,flat=%d>", d->T, d->weight_planes,
-                 d->out_enc == SENGINE_ENC_BITS ? "bits" : "f16", kEpi[plan.mode], flat_layout(d, plan.geo) ? 1 : 0);
+    const int64_t wgs = ((int64_t)plan.p.M + 15) / 16 * (plan.p.F / 64);
+    n = snprintf(buf, len, "smallm<T=%d,planes=%d,out=%s,epi=%s,flat=%d,ch=%d>", d->T, d->weight_planes,
+                 d->out_enc == SENGINE_ENC_BITS ? "bits" : "f16", kEpi[plan.mode], flat_layout(d, plan.geo) ? 1 : 0,
+                 plan.mode != EPI_GENERIC && small_split(wgs, d->T, d->weight_planes) ? 32 : 64);
   } else {
     n = snprintf(buf, len, "direct<T=%d,in=%s,planes=%d,out=%s,flat=%d>", d->T,
                  d->in_enc == SENGINE_ENC_BITS ? "bits" : "f16", d->weight_planes,

@@ -39,12 +39,15 @@ def _bits(x):
 
 SHAPES = [  # T, B, C, H, W, C_out, k, stride
     (4, 1, 64, 9, 7, 64, 3, 1),       # a ragged last position tile, 32-channel workgroups
-    (4, 7, 64, 25, 23, 64, 3, 1),     # 252 workgroups of 64 channels: the last split count
-    (4, 16, 64, 16, 16, 64, 3, 1),    # 256: 64-channel workgroups
+    (4, 8, 64, 16, 16, 64, 3, 1),     # 128 workgroups of 64 channels: the last that run as pairs
+    (4, 1, 64, 43, 48, 64, 3, 1),     # 129: 64-channel workgroups
+    (4, 7, 64, 25, 23, 64, 3, 1),     # 252 and 256: the last of one round
+    (4, 16, 64, 16, 16, 64, 3, 1),
     (1, 2, 64, 5, 5, 128, 1, 1),      # one chunk for eight waves
     (2, 1, 320, 6, 6, 64, 3, 2),      # 45 chunks
     (8, 2, 128, 11, 9, 192, 3, 2),    # two rounds of timesteps
-    (8, 9, 64, 22, 22, 64, 1, 1),     # the same, 64-channel workgroups
+    (8, 9, 64, 22, 22, 64, 1, 1),     # the same, 273 workgroups: pairs with two planes, whole with one
+    (8, 13, 64, 22, 22, 64, 1, 1),    # 394: whole
     (4, 3, 128, 2, 2, 64, 3, 1),      # flat layout (four output pixels)
     (4, 5, 64, 3, 3, 128, 5, 1),      # 5x5 window, mostly padding
 ]
@@ -70,7 +73,7 @@ def test_spread_epilogue_exact(dev, T, B, C, H, W, C_out, k, stride, neuron, sta
 
 
 @pytest.mark.parametrize("res_planes,out_planes", [(1, 2), (2, 2), (3, 5)])
-@pytest.mark.parametrize("T,B,C,H,W,C_out,k,stride", [SHAPES[0], SHAPES[2], SHAPES[5], SHAPES[7]])
+@pytest.mark.parametrize("T,B,C,H,W,C_out,k,stride", [SHAPES[0], SHAPES[4], SHAPES[7], SHAPES[10]])
 def test_spread_residual_planes_exact(dev, T, B, C, H, W, C_out, k, stride, res_planes, out_planes):
     x, w, scale, bias, y = _case(T, B, C, H, W, C_out, k, stride, C + H)
     spec = ops.ConvSpec(T=T, B=B, C_in=C, H=H, W=W, C_out=C_out, KH=k, KW=k, stride=stride, padding=k // 2)
