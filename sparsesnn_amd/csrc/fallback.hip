@@ -18,11 +18,13 @@
 
 namespace sengine {
 
-// 64-row x 64-channel units from which a workgroup takes two of them (each weight fragment read
-// from LDS then feeds two row tiles).  Smaller outputs run one stage's latency after another and
-// want more workgroups: 200 units 18.0 us with one unit each, 21.7 with two; 3,136 units 46.7
-// against 41.4.  Four units measured slower at every size (fewer, longer workgroups in a round).
-constexpr int64_t kDenseWideUnits = 1536;
+// 64-row x 64-channel units per CU from which a workgroup takes two of them (each weight fragment
+// read from LDS then feeds two row tiles).  Smaller outputs run one stage's latency after another and
+// want more workgroups.  3x3, 128 channels in, one unit / two, us: 192 units 8.7 / 10.4, 592 14.2 /
+// 14.8, 800 16.8 / 15.4, 1,200 22.1 / 20.7, 3,136 46.4 / 39.8; two weight planes 592 21.2 / 21.4, 800
+// 25.9 / 22.1; fp16 input 592 20.2 / 23.0, 800 25.6 / 23.9, 1,200 33.7 / 34.7, 2,000 50.6 / 47.3.  Four
+// units measured slower at every size (fewer, longer workgroups in a round).
+constexpr int64_t kDenseWideUnits = 3;
 
 struct DenseParams {
   const uint8_t* in;
@@ -201,7 +203,7 @@ static hipError_t launch_dense(DenseParams& p, int taps, hipStream_t s) {
 template <int IN_ENC, int PLANES, int CW>
 static hipError_t launch_dense_rt(DenseParams& p, int taps, hipStream_t s) {
   const int64_t units = (p.rows + 63) / 64 * (p.F / 64);
-  return units >= kDenseWideUnits ? launch_dense<IN_ENC, PLANES, 2, CW>(p, taps, s)
+  return units >= kDenseWideUnits * device_cus() ? launch_dense<IN_ENC, PLANES, 2, CW>(p, taps, s)
                                   : launch_dense<IN_ENC, PLANES, 1, CW>(p, taps, s);
 }
 

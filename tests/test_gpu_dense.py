@@ -21,6 +21,8 @@ EPS = 2.0 ** -24  # fp32 unit roundoff
     (1, 1, 32, 12, 12, 64, 9, 1, 4, 1),     # more than 64 taps
     (4, 16, 64, 41, 39, 64, 1, 1, 0, 1),    # 1,600 units: two row tiles per wave, ragged last tile
     (4, 10, 256, 25, 25, 256, 3, 1, 1, 1),  # 1,564 units over several output groups
+    (4, 4, 32, 52, 59, 64, 3, 1, 1, 1),     # 767 units: the last with one row tile per wave
+    (4, 4, 96, 55, 56, 64, 3, 1, 1, 1),     # 770: two
 ])
 @pytest.mark.parametrize("in_enc,planes", [(ops.ENC_BITS, 1), (ops.ENC_F16, 1), (ops.ENC_BITS, 2), (ops.ENC_F16, 2)])
 def test_dense_conv_edges(dev, T, B, C, H, W, C_out, k, stride, pad, dil, in_enc, planes):
