@@ -313,15 +313,16 @@ int sengine_amd_ssa_attention(int32_t T, int32_t B, int32_t N, int32_t C, int32_
                               uint32_t* out_bits, hipStream_t stream);
 
 /*
- * Allocation-free spiking self-attention: sengine_amd_ssa_kv followed by
- * sengine_amd_ssa_attend_neuron with the K^T V partial sums in a library-owned device array
- * instead of a caller workspace.  No counterpart in the reference: for callers that cannot
- * allocate (code under HIP graph capture, serving loops, harnesses that forbid hipMalloc).
- * The array holds at most 4,194,304 int32 (16 MiB, T * B * heads * (C/heads)^2 entries; larger
- * calls return -2), every GPU the library runs on keeps one until the process ends, and the
- * call allocates nothing (the array's address is looked up once per device).  All calls on
- * one GPU share the array: calls that overlap on that GPU (other streams, or threads) race.
- * Arguments and results as the two entries above.
+ * Allocation-free spiking self-attention: sengine_amd_ssa_attention without a caller workspace; a
+ * call that is two kernels keeps the K^T V partial sums in a library-owned device array.  No
+ * counterpart in the reference: for callers that cannot allocate (code under HIP graph capture,
+ * serving loops, harnesses that forbid hipMalloc).  The array holds at most 4,194,304 int32 (16 MiB,
+ * T * B * heads * (C/heads)^2 entries; larger calls of either kind return -2), every GPU the library
+ * runs on keeps one until the process ends, and the call allocates nothing (the array's address is
+ * looked up once per device).  All two-kernel calls (sengine_amd_ssa_attention_needs_kv with
+ * workspace 0 returns nonzero) on one GPU share the array: those that overlap on that GPU (other
+ * streams, or threads) race.  One-kernel calls do not touch it.
+ * Arguments and results as sengine_amd_ssa_kv and sengine_amd_ssa_attend_neuron.
  */
 int sengine_amd_ssa_attention_noalloc(int32_t T, int32_t B, int32_t N, int32_t C, int32_t heads, float scale,
                                       int32_t neuron, int32_t hard_reset, float tau, float v_threshold, float v_reset,

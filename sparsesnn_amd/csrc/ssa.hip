@@ -792,7 +792,8 @@ int fused_launch(const SsaParams& p, bool fast, hipStream_t stream) {
   }
 }
 
-// Allocation-free attention: K^T V in a file-scope device array instead of a caller workspace.
+// Allocation-free attention: K^T V in a file-scope device array instead of a caller workspace, for the
+// calls that are two kernels.
 // Each GPU holds its own copy; its address is taken once per device (host code never passes
 // the array's name itself, which on the host is only a stand-in for the symbol).
 constexpr size_t kSsaScratchInts = size_t(1) << 22;  // 16 MiB: T*B*heads*d*d int32 at most
@@ -849,6 +850,9 @@ extern "C" int sengine_amd_ssa_attention_noalloc(int32_t T, int32_t B, int32_t N
   const size_t d = (size_t)(C / heads);
   if ((size_t)T * B * heads * d * d > kSsaScratchInts)
     return set_error(-2, "ssa_attention_noalloc: T * B * heads * (C/heads)^2 exceeds the 4,194,304-entry scratch");
+  if (fused_takes(T, B, N, C / heads, heads, false))  // one kernel: the array is not touched
+    return sengine_amd_ssa_attention(T, B, N, C, heads, scale, neuron, hard_reset, tau, v_threshold, v_reset, q_bits,
+                                     k_bits, v_bits, nullptr, out_bits, stream);
   int32_t* kv = nullptr;
   int rc = scratch_for_current_device(&kv);
   if (rc) return rc;

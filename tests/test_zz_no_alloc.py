@@ -46,3 +46,22 @@ def test_noalloc_attention_refuses_oversize(dev):
     rc, _ = _noalloc(dev, z, z, z, T, B, N, C, heads)
     assert rc == -2
     assert "scratch" in _lib.load().sengine_amd_last_error().decode()
+
+
+def test_noalloc_one_kernel_calls_may_overlap(dev):
+    """Calls that are one kernel share nothing: two streams at a time, other inputs on each."""
+    shapes = [(4, 4, 196, 384, 8), (2, 2, 130, 256, 8)]
+    assert not any(ops.attention_needs_kv(*s) for s in shapes)
+    args = [[_bits(dev, *s[:4], 0.25, 7 * i + j) for j in range(3)] for i, s in enumerate(shapes)]
+    refs = [ops.spiking_self_attention(*a, *s) for a, s in zip(args, shapes)]
+    streams = [torch.cuda.Stream(dev) for _ in shapes]
+    torch.cuda.synchronize()
+    outs = [[], []]
+    for _ in range(20):
+        for i, (a, s) in enumerate(zip(args, shapes)):
+            with torch.cuda.stream(streams[i]):
+                rc, out = _noalloc(dev, *a, *s)
+                assert rc == 0, _lib.load().sengine_amd_last_error().decode()
+                outs[i].append(out)
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, r) for got, r in zip(outs, refs) for o in got)
