@@ -50,6 +50,32 @@ __device__ __forceinline__ void fire_hard4(float& h0, float& h1, float& h2, floa
       : "vcc");
 }
 
+// The same with a soft reset: h -= v_th where it fired (h - 0 elsewhere, which is h).
+__device__ __forceinline__ void fire_soft4(float& h0, float& h1, float& h2, float& h3, float vth, uint32_t& word) {
+  uint64_t s1, s2, s3;
+  float d0, d1, d2, d3;
+  asm("v_cmp_le_f32_e32 vcc, %[th], %[h0]\n\t"
+      "v_cmp_le_f32_e64 %[s1], %[th], %[h1]\n\t"
+      "v_cmp_le_f32_e64 %[s2], %[th], %[h2]\n\t"
+      "v_cmp_le_f32_e64 %[s3], %[th], %[h3]\n\t"
+      "v_cndmask_b32_e32 %[d0], 0, %[thv], vcc\n\t"
+      "v_cndmask_b32_e64 %[d1], 0, %[thv], %[s1]\n\t"
+      "v_cndmask_b32_e64 %[d2], 0, %[thv], %[s2]\n\t"
+      "v_cndmask_b32_e64 %[d3], 0, %[thv], %[s3]\n\t"
+      "v_addc_co_u32_e32 %[w], vcc, %[w], %[w], vcc\n\t"
+      "v_addc_co_u32_e64 %[w], vcc, %[w], %[w], %[s1]\n\t"
+      "v_addc_co_u32_e64 %[w], vcc, %[w], %[w], %[s2]\n\t"
+      "v_addc_co_u32_e64 %[w], vcc, %[w], %[w], %[s3]\n\t"
+      "v_sub_f32_e32 %[h0], %[h0], %[d0]\n\t"
+      "v_sub_f32_e32 %[h1], %[h1], %[d1]\n\t"
+      "v_sub_f32_e32 %[h2], %[h2], %[d2]\n\t"
+      "v_sub_f32_e32 %[h3], %[h3], %[d3]"
+      : [h0] "+v"(h0), [h1] "+v"(h1), [h2] "+v"(h2), [h3] "+v"(h3), [w] "+v"(word), [s1] "=&s"(s1), [s2] "=&s"(s2),
+        [s3] "=&s"(s3), [d0] "=&v"(d0), [d1] "=&v"(d1), [d2] "=&v"(d2), [d3] "=&v"(d3)
+      : [th] "s"(vth), [thv] "v"(vth)
+      : "vcc");
+}
+
 // The spike bits alone (last timestep, membrane not kept).
 __device__ __forceinline__ void fire_only4(float h0, float h1, float h2, float h3, float vth, uint32_t& word) {
   uint64_t s1, s2, s3;

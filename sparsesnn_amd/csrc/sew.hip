@@ -336,6 +336,8 @@ __global__ __launch_bounds__(kStemPix * 16 / CPT) void stem_conv_bn_lds_kernel(S
   }
 }
 
+enum { kStemHard, kStemSoft, kStemDecay };  // neuron of the matrix-core stem
+
 // Stem + neuron on the fp32 matrix cores (v_mfma_f32_16x16x4_f32, 4 taps per instruction):
 // the convolution as a GEMM of channels x (C_ * KH_ * KW_ taps, HWIO order: tap k =
 // (kh * KW + kw) * C + c, zero weights past the last tap) x (output pixels).  Workgroup = (image
@@ -351,11 +353,13 @@ __global__ __launch_bounds__(kStemPix * 16 / CPT) void stem_conv_bn_lds_kernel(S
 // register, and a 4 x 4 nibble transpose among the lanes of a pixel (two butterfly steps) leaves
 // lane l with the whole channel words of one timestep: one store per tile pair for four steps.
 // The products are summed in a different order than the FMA kernels', so outputs agree to fp32
-// rounding.  FASTN: hard-reset LIF with power-of-two 1/tau and 1 - 1/tau, or hard-reset IF, whose
-// charge is one fma (IF: v * 1 + x, the same single rounding as v + x); else the generic neuron.
+// rounding.  NMODE: kStemHard / kStemSoft where the charge is one fma -- LIF with power-of-two 1/tau and
+// 1 - 1/tau, or IF (v * 1 + x, the same single rounding as v + x) -- with a hard or soft reset; kStemDecay
+// a LIF of any other tau, whose v * decay and x / tau are rounded on their own.  SHORT: T < 4, the steps
+// that there are (in the same kernel their path cost the others 2 %).
 // 7x7/2 224x224, 64 channels, T = 4, fp32 output kept: 8 images 44.0 -> 34.6 us, 32 images
 // 114.9 -> 110.1; 3x3 224x224, spikes only, 32 images: 171.9 -> 124.4.
-template <int C_, int KH_, int KW_, int CT, int NCG, bool FASTN, int NB>
+template <int C_, int KH_, int KW_, int CT, int NCG, int NMODE, bool SHORT, int NB>
 __global__ __launch_bounds__(256) void stem_mfma_kernel(StemParams p) {
   constexpr int NT = 256;
   constexpr int K = C_ * KH_ * KW_;
@@ -449,33 +453,37 @@ __global__ __launch_bounds__(256) void stem_mfma_kernel(StemParams p) {
       if (p.out && st)
         *reinterpret_cast<out4_t*>(p.out + opix * p.F + ch0 + 16 * c + 4 * q) =
             out4_t{xo[c][0], xo[c][1], xo[c][2], xo[c][3]};
-      if (fold) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) xo[c][r] *= p.np.rtau;  // exact
+      for (int r = 0; r < 4; ++r) {
+        if (NMODE == kStemDecay) xo[c][r] = __fdiv_rn(xo[c][r], p.np.tau);  // the same input at every step
+        else if (fold) xo[c][r] *= p.np.rtau;  // exact
       }
     }
     for (int t0 = 0; t0 < p.T; t0 += 4) {
       uint32_t nib[CT];
 #pragma unroll
       for (int c = 0; c < CT; ++c) nib[c] = 0u;
-#pragma unroll
-      for (int k = 0; k < 4; ++k)  // steps past T run and are not stored
+      auto step = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int c = 0; c < CT; ++c) {
-          if (FASTN) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) v[c][r] = __builtin_fmaf(v[c][r], dec, xo[c][r]);
+          for (int r = 0; r < 4; ++r)
+            v[c][r] = NMODE == kStemDecay ? __fadd_rn(__fmul_rn(v[c][r], dec), xo[c][r])
+                                          : __builtin_fmaf(v[c][r], dec, xo[c][r]);
+          if (NMODE == kStemHard || (NMODE == kStemDecay && p.np.hard_reset))
             fire_hard4(v[c][3], v[c][2], v[c][1], v[c][0], p.np.vth, p.np.vreset, nib[c]);
-          } else {
-#pragma unroll
-            for (int r = 3; r >= 0; --r) {
-              const float h = neuron_charge(p.np, v[c][r], xo[c][r]);
-              const bool spike = h >= p.np.vth;
-              v[c][r] = neuron_reset(p.np, h, spike);
-              nib[c] = 2 * nib[c] + (uint32_t)spike;
-            }
-          }
+          else
+            fire_soft4(v[c][3], v[c][2], v[c][1], v[c][0], p.np.vth, nib[c]);
         }
+      };
+      if (SHORT) {
+        for (int k = 0; k < p.T; ++k) step();
+#pragma unroll
+        for (int c = 0; c < CT; ++c) nib[c] <<= 4 * (4 - p.T);
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) step();  // steps past T run and are not stored
+      }
       // nib: step t0 + k in nibble 3 - k.  Lane group q ends with step t0 + 3 - q, the nibble of
       // source group g at bits 4g of the tile's 16.
       const int t = t0 + 3 - q;
@@ -869,14 +877,14 @@ static int64_t stem_staged(const StemParams& p, int pix) {
 
 // Launch geometry of stem_mfma_kernel<..., NB>: workgroups, the rounds the chip needs for
 // them at the occupancy the kernel reaches (resident workgroups per CU x CUs), and its LDS.
-template <int K_, int CT, int NCG, bool FASTN, int NB>
+template <int K_, int CT, int NCG, int NMODE, bool SHORT, int NB>
 static void stem_mfma_shape(const StemParams& p, int cus, int64_t& wgs, int64_t& rounds, size_t& lds) {
   constexpr int PIX = 16 * NB * (4 / NCG);
   lds = (size_t)(stem_staged(p, PIX) + 4 * ((3 * K_ * K_ + 3) / 4)) * sizeof(float);  // + tap offsets
   wgs = (int64_t)p.N * ((p.OH * p.OW + PIX - 1) / PIX);
   int per_cu = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(
-                                                       &stem_mfma_kernel<3, K_, K_, CT, NCG, FASTN, NB>),
+                                                       &stem_mfma_kernel<3, K_, K_, CT, NCG, NMODE, SHORT, NB>),
                                                    256, lds) != hipSuccess ||
       per_cu < 1)
     per_cu = 1;
@@ -887,7 +895,7 @@ static void stem_mfma_shape(const StemParams& p, int cus, int64_t& wgs, int64_t&
 // Pixels per workgroup (16 NB * 4 / NCG): the fewest pixel-block rounds over the chip, weighing a
 // round by its workgroup's pixels plus 64 for what every workgroup pays (staging, weights): without
 // that term the 32-image 7x7 stem took seven rounds of 128 pixels (117.8 us) over four of 256 (110.1).
-template <int K_, int CT, int NCG, bool FASTN>
+template <int K_, int CT, int NCG, int NMODE, bool SHORT>
 static int launch_stem_mfma(const StemParams& p, hipStream_t stream) {
   constexpr int S = 4 / NCG;  // pixel sets per workgroup
   constexpr int NL = 16 / S, NM = 12 / S, NS = 8 / S;  // 256, 192 or 128 pixels
@@ -897,9 +905,9 @@ static int launch_stem_mfma(const StemParams& p, hipStream_t stream) {
     cus = 256;
   int64_t wl, rl, wm, rm, ws, rs;
   size_t ll, lm, ls;
-  stem_mfma_shape<K_, CT, NCG, FASTN, NL>(p, cus, wl, rl, ll);
-  stem_mfma_shape<K_, CT, NCG, FASTN, NM>(p, cus, wm, rm, lm);
-  stem_mfma_shape<K_, CT, NCG, FASTN, NS>(p, cus, ws, rs, ls);
+  stem_mfma_shape<K_, CT, NCG, NMODE, SHORT, NL>(p, cus, wl, rl, ll);
+  stem_mfma_shape<K_, CT, NCG, NMODE, SHORT, NM>(p, cus, wm, rm, lm);
+  stem_mfma_shape<K_, CT, NCG, NMODE, SHORT, NS>(p, cus, ws, rs, ls);
   int nb = 16;
   int64_t best = rl * (16 + 4);
   if (rm * (12 + 4) < best) { nb = 12; best = rm * (12 + 4); }
@@ -910,11 +918,11 @@ static int launch_stem_mfma(const StemParams& p, hipStream_t stream) {
   }
   const dim3 block(256);
   if (nb == 16)
-    hipLaunchKernelGGL((stem_mfma_kernel<3, K_, K_, CT, NCG, FASTN, NL>), dim3((unsigned)wl), block, ll, stream, p);
+    hipLaunchKernelGGL((stem_mfma_kernel<3, K_, K_, CT, NCG, NMODE, SHORT, NL>), dim3((unsigned)wl), block, ll, stream, p);
   else if (nb == 12)
-    hipLaunchKernelGGL((stem_mfma_kernel<3, K_, K_, CT, NCG, FASTN, NM>), dim3((unsigned)wm), block, lm, stream, p);
+    hipLaunchKernelGGL((stem_mfma_kernel<3, K_, K_, CT, NCG, NMODE, SHORT, NM>), dim3((unsigned)wm), block, lm, stream, p);
   else
-    hipLaunchKernelGGL((stem_mfma_kernel<3, K_, K_, CT, NCG, FASTN, NS>), dim3((unsigned)ws), block, ls, stream, p);
+    hipLaunchKernelGGL((stem_mfma_kernel<3, K_, K_, CT, NCG, NMODE, SHORT, NS>), dim3((unsigned)ws), block, ls, stream, p);
   return (int)hipGetLastError();
 }
 
@@ -992,11 +1000,18 @@ extern "C" int sengine_amd_stem_conv_bn_neuron(const sengine_conv_lif_desc* d, c
   // The matrix-core kernel for the 3-channel 7x7 and 3x3 stems of 32 or 64 channels (one
   // wave per 16 channels); SENGINE_AMD_STEM_MFMA=0 keeps the FMA kernel.
   if (p.C == 3 && p.KH == p.KW && (p.KW == 7 || p.KW == 3) && (p.F == 32 || p.F == 64) && env_stem_mfma()) {
-    const bool fast = p.np.hard_reset && (p.np.neuron == SENGINE_NEURON_IF ||
-                                          (p.np.neuron == SENGINE_NEURON_LIF && p.np.pow2));
-#define SENGINE_STEM_CASE(K, FF, CT, NCG) \
-  if (p.KW == K && p.F == FF)             \
-    return fast ? launch_stem_mfma<K, CT, NCG, true>(p, stream) : launch_stem_mfma<K, CT, NCG, false>(p, stream);
+    const bool one_fma = p.np.neuron == SENGINE_NEURON_IF || (p.np.neuron == SENGINE_NEURON_LIF && p.np.pow2);
+    const int mode = !one_fma ? kStemDecay : p.np.hard_reset ? kStemHard : kStemSoft;
+#define SENGINE_STEM_MODE(K, CT, NCG, M)                                        \
+  if (mode == M)                                                                 \
+    return p.T < 4 ? launch_stem_mfma<K, CT, NCG, M, true>(p, stream)            \
+                   : launch_stem_mfma<K, CT, NCG, M, false>(p, stream);
+#define SENGINE_STEM_CASE(K, FF, CT, NCG)          \
+  if (p.KW == K && p.F == FF) {                    \
+    SENGINE_STEM_MODE(K, CT, NCG, kStemHard)       \
+    SENGINE_STEM_MODE(K, CT, NCG, kStemSoft)       \
+    SENGINE_STEM_MODE(K, CT, NCG, kStemDecay)      \
+  }
     // channel tiles per wave: all of them where a tile's weights take few registers (3x3: 7),
     // two for the 7x7 stem's 37
     SENGINE_STEM_CASE(7, 64, 2, 2)
@@ -1004,6 +1019,7 @@ extern "C" int sengine_amd_stem_conv_bn_neuron(const sengine_conv_lif_desc* d, c
     SENGINE_STEM_CASE(3, 64, 4, 1)
     SENGINE_STEM_CASE(3, 32, 2, 1)
 #undef SENGINE_STEM_CASE
+#undef SENGINE_STEM_MODE
   }
   const int64_t blocks = pblocks * (p.F / 16);
   if (p.KW == 7)

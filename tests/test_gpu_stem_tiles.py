@@ -17,6 +17,9 @@ pytestmark = pytest.mark.gpu
     (3, 23, 130, 64, 3, 2, "lif", 1, None, 2.0),  # one step, soft reset, wide rows
     (2, 31, 31, 32, 3, 1, "if", 6, 0.25, 2.0),   # two tiles, nonzero reset value
     (1, 40, 24, 32, 7, 2, "lif", 5, 0.0, 1.5),   # general decay
+    (2, 29, 45, 64, 7, 2, "lif", 8, None, 2.0),  # soft reset over full groups of four steps
+    (1, 12, 19, 32, 3, 1, "if", 7, None, 2.0),   # and a rest of three
+    (1, 16, 16, 64, 3, 1, "lif", 6, None, 3.0),  # soft reset, general decay, a rest of two
 ])
 def test_stem_blocks(dev, env, nb, B, H, W, C_out, K, S, neuron, T, v_reset, tau):
     env("SENGINE_AMD_STEM_NB", nb)
