@@ -357,10 +357,12 @@ enum { kStemHard, kStemSoft, kStemDecay };  // neuron of the matrix-core stem
 // 1 - 1/tau, or IF (v * 1 + x, the same single rounding as v + x) -- with a hard or soft reset; kStemDecay
 // a LIF of any other tau, whose v * decay and x / tau are rounded on their own.  SHORT: T < 4, the steps
 // that there are (in the same kernel their path cost the others 2 %).
-// 7x7/2 224x224, 64 channels, T = 4, fp32 output kept: 8 images 44.0 -> 34.6 us, 32 images
-// 114.9 -> 110.1; 3x3 224x224, spikes only, 32 images: 171.9 -> 124.4.
+// 7x7/2 224x224, 64 channels, T = 4, fp32 output kept: 8 images 44.0 -> 34.1 us, 32 images 115.1 ->
+// 104.7; 3x3 224x224, spikes only, 32 images: 170.7 -> 128.7.  The 128-pixel 7x7 form, held to three
+// waves per SIMD, takes 136 registers (180 left to itself): 32 images, spikes only, 115 -> 99.5 us.
 template <int C_, int KH_, int KW_, int CT, int NCG, int NMODE, bool SHORT, int NB>
-__global__ __launch_bounds__(256) void stem_mfma_kernel(StemParams p) {
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(KW_ == 7 && NB <= 4 ? 3 : 1))) void stem_mfma_kernel(StemParams p) {
   constexpr int NT = 256;
   constexpr int K = C_ * KH_ * KW_;
   constexpr int KS = (K + 3) / 4;
@@ -875,10 +877,14 @@ static int64_t stem_staged(const StemParams& p, int pix) {
   return (int64_t)p.C * ((orows - 1) * p.SH + p.KH) * (p.W + 2 * p.PW);
 }
 
-// Launch geometry of stem_mfma_kernel<..., NB>: workgroups, the rounds the chip needs for
-// them at the occupancy the kernel reaches (resident workgroups per CU x CUs), and its LDS.
+// Workgroups of stem_mfma_kernel<..., NB>, its LDS (returned by reference), and an estimate of its time.
+// A workgroup costs its 16-pixel sets plus 4 for what every one pays (staging, weights); o of them on a
+// CU take 1.5 + o times as long each (7x7: three against two 1.22 times, 3x3: five against four 1.3); a
+// grid larger than the chip ends in workgroups that run about alone.  Within 0.4 % of the best of the
+// three block sizes over 268 shapes (worst 17 %).  Whole rounds in place of this took 128 pixels for
+// the 3x3, 32-channel stem (five on a CU): 77 us at T = 1, 32 images of 224x224, against 62 with 256.
 template <int K_, int CT, int NCG, int NMODE, bool SHORT, int NB>
-static void stem_mfma_shape(const StemParams& p, int cus, int64_t& wgs, int64_t& rounds, size_t& lds) {
+static double stem_mfma_cost(const StemParams& p, int cus, int64_t& wgs, size_t& lds) {
   constexpr int PIX = 16 * NB * (4 / NCG);
   lds = (size_t)(stem_staged(p, PIX) + 4 * ((3 * K_ * K_ + 3) / 4)) * sizeof(float);  // + tap offsets
   wgs = (int64_t)p.N * ((p.OH * p.OW + PIX - 1) / PIX);
@@ -889,29 +895,25 @@ static void stem_mfma_shape(const StemParams& p, int cus, int64_t& wgs, int64_t&
       per_cu < 1)
     per_cu = 1;
   const int64_t slots = (int64_t)per_cu * cus;
-  rounds = (wgs + slots - 1) / slots;
+  const double one = PIX / 16 + 4;
+  return wgs <= slots ? one * (1.5 + (double)((wgs + cus - 1) / cus))
+                      : one * ((1.5 + per_cu) * (double)wgs / (double)slots + 2.5);
 }
 
-// Pixels per workgroup (16 NB * 4 / NCG): the fewest pixel-block rounds over the chip, weighing a
-// round by its workgroup's pixels plus 64 for what every workgroup pays (staging, weights): without
-// that term the 32-image 7x7 stem took seven rounds of 128 pixels (117.8 us) over four of 256 (110.1).
+// Pixels per workgroup (16 NB * 4 / NCG): 256, 192 or 128, whichever that estimate favours.
 template <int K_, int CT, int NCG, int NMODE, bool SHORT>
 static int launch_stem_mfma(const StemParams& p, hipStream_t stream) {
   constexpr int S = 4 / NCG;  // pixel sets per workgroup
   constexpr int NL = 16 / S, NM = 12 / S, NS = 8 / S;  // 256, 192 or 128 pixels
-  int dev = 0, cus = 256;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
-                                               hipSuccess)
-    cus = 256;
-  int64_t wl, rl, wm, rm, ws, rs;
+  const int cus = device_cus();
+  int64_t wl, wm, ws;
   size_t ll, lm, ls;
-  stem_mfma_shape<K_, CT, NCG, NMODE, SHORT, NL>(p, cus, wl, rl, ll);
-  stem_mfma_shape<K_, CT, NCG, NMODE, SHORT, NM>(p, cus, wm, rm, lm);
-  stem_mfma_shape<K_, CT, NCG, NMODE, SHORT, NS>(p, cus, ws, rs, ls);
+  double best = stem_mfma_cost<K_, CT, NCG, NMODE, SHORT, NL>(p, cus, wl, ll);
+  const double cm = stem_mfma_cost<K_, CT, NCG, NMODE, SHORT, NM>(p, cus, wm, lm);
+  const double cs = stem_mfma_cost<K_, CT, NCG, NMODE, SHORT, NS>(p, cus, ws, ls);
   int nb = 16;
-  int64_t best = rl * (16 + 4);
-  if (rm * (12 + 4) < best) { nb = 12; best = rm * (12 + 4); }
-  if (rs * (8 + 4) < best) nb = 8;
+  if (cm < best) { nb = 12; best = cm; }
+  if (cs < best) nb = 8;
   if (const char* e = getenv("SENGINE_AMD_STEM_NB")) {
     const int f = atoi(e);
     if (f == 16 || f == 12 || f == 8) nb = f;
