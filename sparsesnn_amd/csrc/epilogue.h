@@ -25,69 +25,69 @@ enum { EPI_GENERIC = 0, EPI_LIF_HARD = 1, EPI_IF_HARD = 2, EPI_SHORTCUT = 3, EPI
 // compiler's form needs a separate select to materialise the bit.
 //
 // gfx950 wants two wait states between a VALU write of VCC or an SGPR and a VALU read of it, and the
-// compiler puts none inside an asm block: every compare has its own SGPR pair and three other
-// instructions between it and its first reader.  (One neuron at a time through VCC, as these blocks
-// were, has none or one.)  Filling the waits with neighbours costs no issue slots, where the
-// compiler's s_nop after each compare would.
+// compiler puts none inside an asm block: two other instructions stand between every compare and its
+// first reader.  (One neuron at a time through VCC, as these blocks were, left none or one.)  Filling
+// the waits with neighbours costs no issue slots, where the compiler's s_nop after each compare would.
+// The first and last neuron take VCC and the short encodings: with an SGPR pair for each of them the
+// VALU-bound 256->1024 14x14 1x1 layer took 13.4 us, 13.1 so.
 __device__ __forceinline__ void fire_hard4(float& h0, float& h1, float& h2, float& h3, float vth, float vreset,
                                            uint32_t& word) {
-  uint64_t s1, s2, s3;
+  uint64_t s1, s2;
   asm("v_cmp_le_f32_e32 vcc, %[th], %[h0]\n\t"
       "v_cmp_le_f32_e64 %[s1], %[th], %[h1]\n\t"
       "v_cmp_le_f32_e64 %[s2], %[th], %[h2]\n\t"
-      "v_cmp_le_f32_e64 %[s3], %[th], %[h3]\n\t"
       "v_cndmask_b32_e32 %[h0], %[h0], %[vr], vcc\n\t"
+      "v_addc_co_u32_e32 %[w], vcc, %[w], %[w], vcc\n\t"
+      "v_cmp_le_f32_e32 vcc, %[th], %[h3]\n\t"
       "v_cndmask_b32_e64 %[h1], %[h1], %[vr], %[s1]\n\t"
       "v_cndmask_b32_e64 %[h2], %[h2], %[vr], %[s2]\n\t"
-      "v_cndmask_b32_e64 %[h3], %[h3], %[vr], %[s3]\n\t"
-      "v_addc_co_u32_e32 %[w], vcc, %[w], %[w], vcc\n\t"
-      "v_addc_co_u32_e64 %[w], vcc, %[w], %[w], %[s1]\n\t"
-      "v_addc_co_u32_e64 %[w], vcc, %[w], %[w], %[s2]\n\t"
-      "v_addc_co_u32_e64 %[w], vcc, %[w], %[w], %[s3]"
-      : [h0] "+v"(h0), [h1] "+v"(h1), [h2] "+v"(h2), [h3] "+v"(h3), [w] "+v"(word), [s1] "=&s"(s1), [s2] "=&s"(s2),
-        [s3] "=&s"(s3)
+      "v_cndmask_b32_e32 %[h3], %[h3], %[vr], vcc\n\t"
+      "v_addc_co_u32_e64 %[w], %[s1], %[w], %[w], %[s1]\n\t"
+      "v_addc_co_u32_e64 %[w], %[s2], %[w], %[w], %[s2]\n\t"
+      "v_addc_co_u32_e32 %[w], vcc, %[w], %[w], vcc"
+      : [h0] "+v"(h0), [h1] "+v"(h1), [h2] "+v"(h2), [h3] "+v"(h3), [w] "+v"(word), [s1] "=&s"(s1), [s2] "=&s"(s2)
       : [th] "s"(vth), [vr] "v"(vreset)
       : "vcc");
 }
 
 // The same with a soft reset: h -= v_th where it fired (h - 0 elsewhere, which is h).
 __device__ __forceinline__ void fire_soft4(float& h0, float& h1, float& h2, float& h3, float vth, uint32_t& word) {
-  uint64_t s1, s2, s3;
+  uint64_t s1, s2;
   float d0, d1, d2, d3;
   asm("v_cmp_le_f32_e32 vcc, %[th], %[h0]\n\t"
       "v_cmp_le_f32_e64 %[s1], %[th], %[h1]\n\t"
       "v_cmp_le_f32_e64 %[s2], %[th], %[h2]\n\t"
-      "v_cmp_le_f32_e64 %[s3], %[th], %[h3]\n\t"
       "v_cndmask_b32_e32 %[d0], 0, %[thv], vcc\n\t"
+      "v_addc_co_u32_e32 %[w], vcc, %[w], %[w], vcc\n\t"
+      "v_cmp_le_f32_e32 vcc, %[th], %[h3]\n\t"
       "v_cndmask_b32_e64 %[d1], 0, %[thv], %[s1]\n\t"
       "v_cndmask_b32_e64 %[d2], 0, %[thv], %[s2]\n\t"
-      "v_cndmask_b32_e64 %[d3], 0, %[thv], %[s3]\n\t"
+      "v_cndmask_b32_e32 %[d3], 0, %[thv], vcc\n\t"
+      "v_addc_co_u32_e64 %[w], %[s1], %[w], %[w], %[s1]\n\t"
+      "v_addc_co_u32_e64 %[w], %[s2], %[w], %[w], %[s2]\n\t"
       "v_addc_co_u32_e32 %[w], vcc, %[w], %[w], vcc\n\t"
-      "v_addc_co_u32_e64 %[w], vcc, %[w], %[w], %[s1]\n\t"
-      "v_addc_co_u32_e64 %[w], vcc, %[w], %[w], %[s2]\n\t"
-      "v_addc_co_u32_e64 %[w], vcc, %[w], %[w], %[s3]\n\t"
       "v_sub_f32_e32 %[h0], %[h0], %[d0]\n\t"
       "v_sub_f32_e32 %[h1], %[h1], %[d1]\n\t"
       "v_sub_f32_e32 %[h2], %[h2], %[d2]\n\t"
       "v_sub_f32_e32 %[h3], %[h3], %[d3]"
       : [h0] "+v"(h0), [h1] "+v"(h1), [h2] "+v"(h2), [h3] "+v"(h3), [w] "+v"(word), [s1] "=&s"(s1), [s2] "=&s"(s2),
-        [s3] "=&s"(s3), [d0] "=&v"(d0), [d1] "=&v"(d1), [d2] "=&v"(d2), [d3] "=&v"(d3)
+        [d0] "=&v"(d0), [d1] "=&v"(d1), [d2] "=&v"(d2), [d3] "=&v"(d3)
       : [th] "s"(vth), [thv] "v"(vth)
       : "vcc");
 }
 
 // The spike bits alone (last timestep, membrane not kept).
 __device__ __forceinline__ void fire_only4(float h0, float h1, float h2, float h3, float vth, uint32_t& word) {
-  uint64_t s1, s2, s3;
+  uint64_t s1, s2;
   asm("v_cmp_le_f32_e32 vcc, %[th], %[h0]\n\t"
       "v_cmp_le_f32_e64 %[s1], %[th], %[h1]\n\t"
       "v_cmp_le_f32_e64 %[s2], %[th], %[h2]\n\t"
-      "v_cmp_le_f32_e64 %[s3], %[th], %[h3]\n\t"
       "v_addc_co_u32_e32 %[w], vcc, %[w], %[w], vcc\n\t"
-      "v_addc_co_u32_e64 %[w], vcc, %[w], %[w], %[s1]\n\t"
-      "v_addc_co_u32_e64 %[w], vcc, %[w], %[w], %[s2]\n\t"
-      "v_addc_co_u32_e64 %[w], vcc, %[w], %[w], %[s3]"
-      : [w] "+v"(word), [s1] "=&s"(s1), [s2] "=&s"(s2), [s3] "=&s"(s3)
+      "v_cmp_le_f32_e32 vcc, %[th], %[h3]\n\t"
+      "v_addc_co_u32_e64 %[w], %[s1], %[w], %[w], %[s1]\n\t"
+      "v_addc_co_u32_e64 %[w], %[s2], %[w], %[w], %[s2]\n\t"
+      "v_addc_co_u32_e32 %[w], vcc, %[w], %[w], vcc"
+      : [w] "+v"(word), [s1] "=&s"(s1), [s2] "=&s"(s2)
       : [h0] "v"(h0), [h1] "v"(h1), [h2] "v"(h2), [h3] "v"(h3), [th] "s"(vth)
       : "vcc");
 }
