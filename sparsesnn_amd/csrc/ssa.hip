@@ -18,6 +18,8 @@
 //                      from bits, one fp32 accumulator), the neuron over T in
 //                      registers, 16 output channels of a token assembled across lanes
 //                      and stored as one u16.
+//   ssa_fused_kernel:  both in one workgroup per (b, head), K^T V in LDS only; fused_takes
+//                      says which calls it gets.
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -409,9 +411,9 @@ __global__ __launch_bounds__(256) void ssa_attend_kernel(SsaParams p, int splits
 //   channel masks, and lane i adds popcount(K_i & V_j) for every j to registers, the V masks read
 //   back as LDS broadcasts.  The waves of a timestep meet in LDS by integer atomics (exact).
 //   Q (K^T V): the sums become fp16 pieces in LDS as in ssa_attend_kernel, and each wave walks
-//   16-token tiles: the products of all T steps first (exact in any order), then the neuron with its
-//   spikes shifted into nibbles; a 4 x 4 nibble transpose among the four lanes of a token gives each
-//   of them the channel words of one timestep, one store for four steps.
+//   16-token tiles, step by step: a step's products, then its neuron, the spikes shifted into nibbles;
+//   after four steps a 4 x 4 nibble transpose among the four lanes of a token gives each of them the
+//   channel words of one timestep, one store for the four.
 //
 // Bound by VALU work (transposes, popcounts, the neuron); a (b, head) has little of it, so the launch
 // and the phases' latencies count at small N.  32 images, 8 heads of 48, T = 4: 196 tokens
